@@ -8,8 +8,8 @@ hiprtc-compiled kernel per fused group). The input is resident in HBM before
 timing; each step re-evaluates the 200-generation DAG from that input.
 
 Prints one JSON line: value = cell-generations per second (whole job), with
-the roofline of the dominant kernel (one generation over all blocks, 2 bytes
-of algorithmic HBM traffic per cell: 1 read + 1 write) and a CPU baseline
+the roofline of the dominant kernel (the generations on the bit-packed raster;
+with a forced tile shape one generation over all blocks) and a CPU baseline
 (the oracle's restatement, timed on a bounded sample on the host cores).
 """
 import argparse
@@ -22,6 +22,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+VALU_PEAK_GIPS = 614.4  # 256 CUs x 4 SIMDs, one wavefront instruction per 4 cycles at 2.4 GHz
 
 
 def life_script(M, state, gens):
@@ -622,6 +623,23 @@ def hillshade_bench(M, side=4096, block=512, reps=5, cpu=True):
     return {"workload": "hillshade %dx%d f32, blocks %dx%d" % (side, side, block, block), **out}
 
 
+def bit_chain_roofline(kt, kname, side, gens):
+    """The step kernel of a bit chain (the generations on the bit-packed raster) against VALU issue: 24
+    instructions per 32 cells and generation, 64 lanes an instruction; the rows and columns that
+    neighbouring wavefronts compute twice are not counted."""
+    launches = {k.rsplit("_", 1)[1]: v["count"] for k, v in kt.items() if k.startswith("bit_")}
+    steps = kt[kname]["count"]
+    if len(kt) != 3 or launches.get("pack") != 1 or launches.get("unpack") != 1 or steps != -(-gens // 8):
+        raise SystemExit("bench.py: the profiled step launched %s, expected one bit chain"
+                         % {k: v["count"] for k, v in kt.items()})
+    per = -(-side // 32) * side * 24.0 / 64 * gens / steps  # wavefront instructions of a launch
+    ms = kt[kname]["total_ms"] / steps
+    return {"bound": "valu", "achieved": round(per / ms / 1e6, 1), "peak": VALU_PEAK_GIPS, "unit": "G wave-instr/s",
+            "frac": round(per / ms / 1e6 / VALU_PEAK_GIPS, 4), "kernel": kname, "kernel_avg_ms": round(ms, 5),
+            "launches": steps, "generations_per_launch": round(gens / steps, 2),
+            "kernels_ms": {k.rsplit("_", 1)[1]: round(v["total_ms"], 4) for k, v in kt.items()}}
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -634,7 +652,8 @@ def main():
     ap.add_argument("--graph", type=int, default=1)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--plain-gens", type=int, default=8, help="generations timed once in the plain form")
-    ap.add_argument("--tune", type=int, default=1, help="autotune the tile shape before timing")
+    ap.add_argument("--tune", type=int, default=0,
+                    help="autotune the tile shape of the per-generation kernel (the bit chain has none)")
     ap.add_argument("--tile", default="",
                     help="TX,TY,VX[,PF[,ST[,W]]] tile shape of the Life kernel (implies --tune 0)")
     ap.add_argument("--chunk-tiles", type=int, default=0,
@@ -730,9 +749,8 @@ def main():
     cells = args.side * args.side
     value = cells * args.gens / (wall / args.steps) / 1e9
 
-    # roofline of the dominant kernel (one generation over all blocks), timed
-    # with HIP events around each launch on the compute stream (one extra,
-    # non-graph evaluation after the timed steps)
+    # roofline of the dominant kernel, timed with HIP events around each launch
+    # on the compute stream (one extra, non-graph evaluation after the timed steps)
     M.set_option("graph", 0)
     M.set_option("profile", 1)
     M.kernel_times()
@@ -741,26 +759,33 @@ def main():
     M.set_option("profile", 0)
     M.set_option("graph", args.graph)
     kname, krec = max(kt.items(), key=lambda kv: kv[1]["total_ms"])
-    # every generation is one launch of one kernel: anything else means a
-    # generation ran another kernel (or none) and the roofline would not be
-    # the step's
-    if len(kt) != 1 or krec["count"] != args.gens:
-        raise SystemExit("bench.py: the profiled step launched %s, expected %d launches of one kernel"
-                         % ({k: v["count"] for k, v in kt.items()}, args.gens))
-    # HBM bytes per launch of this kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE
-    # passes scaled by a copy kernel of known size (profiles/life_hbm_traffic.json)
-    traffic = None
-    try:
-        with open(os.path.join(ROOT, "profiles", "life_hbm_traffic.json")) as f:
-            tr = json.load(f)
-        if kname in tr.get("kernels", {}):
-            traffic = tr["kernels"][kname]["bytes_per_launch"]
-    except (OSError, ValueError, KeyError):
-        pass
     launches = krec["count"]
     kern_ms = krec["total_ms"] / krec["count"]
-    alg_bytes = 2.0 * cells  # one U8 read + one U8 write per cell and generation
-    achieved = alg_bytes / (kern_ms * 1e-3) / 1e9
+    if kname.startswith("bit_"):
+        roofline = bit_chain_roofline(kt, kname, args.side, args.gens)
+    else:
+        # every generation is one launch of one kernel: anything else means a
+        # generation ran another kernel (or none) and the roofline would not be
+        # the step's
+        if len(kt) != 1 or launches != args.gens:
+            raise SystemExit("bench.py: the profiled step launched %s, expected %d launches of one kernel"
+                             % ({k: v["count"] for k, v in kt.items()}, args.gens))
+        # HBM bytes per launch of this kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE
+        # passes scaled by a copy kernel of known size (profiles/life_hbm_traffic.json)
+        traffic = None
+        try:
+            with open(os.path.join(ROOT, "profiles", "life_hbm_traffic.json")) as f:
+                tr = json.load(f)
+            if kname in tr.get("kernels", {}):
+                traffic = tr["kernels"][kname]["bytes_per_launch"]
+        except (OSError, ValueError, KeyError):
+            pass
+        alg_bytes = 2.0 * cells  # one U8 read + one U8 write per cell and generation
+        achieved = alg_bytes / (kern_ms * 1e-3) / 1e9
+        roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                    "kernel": kname, "kernel_avg_ms": round(kern_ms, 5), "kernel_min_ms": round(krec["min_ms"], 5),
+                    "launches": launches, "algorithmic_bytes_per_launch": int(alg_bytes)}
     host = M.stats()
     res = {
         "metric": "Life cell-generations/s (fused focal+local group, 200 generations)",
@@ -778,10 +803,7 @@ def main():
         "config": {"workload": "game-of-life %dx%d u8 Bernoulli(0.3) seed 1, %d generations, blocks %dx%d"
                                % (args.side, args.side, args.gens, bs[0], bs[1]),
                    "form": args.form, "graph": bool(args.graph)},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": kname, "kernel_avg_ms": round(kern_ms, 5), "kernel_min_ms": round(krec["min_ms"], 5),
-                     "launches": launches, "algorithmic_bytes_per_launch": int(alg_bytes)},
+        "roofline": roofline,
         "device_ms_per_step": round(min(dev_ms), 3),
         "tuned_tile": tuned,
         "host_ms": {"fuse": round(host["ms_fuse"], 1), "codegen_compile": round(host["ms_codegen"], 1),

@@ -1,5 +1,6 @@
 #include "codegen.hpp"
 #include "dev.hpp"
+#include "runtime.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -1005,6 +1006,153 @@ KernelSpec generate_kernel(const Group& g, const std::vector<Node*>& d2_outs, Ti
   ks.signature = ks.source;
   g_local = nullptr;
   return ks;
+}
+
+// ---- bit rules ----------------------------------------------------------------------
+
+namespace {
+
+// The boolean function given by its values `t` ('0', '1', 'x' for inputs that
+// cannot occur) over the variables vars[k..], as an expression: split on one
+// variable after the other, halves that agree merged.
+std::string bool_expr(const std::string& t, const std::vector<std::string>& vars, size_t k) {
+  bool zero = true, one = true;
+  for (char c : t) { zero &= c != '1'; one &= c != '0'; }
+  if (zero) return "0";
+  if (one) return "1";
+  const std::string lo = t.substr(0, t.size() / 2), hi = t.substr(t.size() / 2);
+  bool same = true;
+  std::string both = lo;
+  for (size_t i = 0; i < lo.size(); i++) {
+    if (lo[i] != 'x' && hi[i] != 'x' && lo[i] != hi[i]) same = false;
+    if (lo[i] == 'x') both[i] = hi[i];
+  }
+  if (same) return bool_expr(both, vars, k + 1);
+  const std::string v = vars[k], l = bool_expr(lo, vars, k + 1), h = bool_expr(hi, vars, k + 1);
+  if (l == "0") return h == "1" ? v : "(" + v + " & " + h + ")";
+  if (l == "1") return h == "0" ? "~" + v : "(~" + v + " | " + h + ")";
+  if (h == "0") return "(~" + v + " & " + l + ")";
+  if (h == "1") return "(" + v + " | " + l + ")";
+  return "mx::bit_sel(" + v + ", " + h + ", " + l + ")";
+}
+
+}  // namespace
+
+BitRule bit_rule(const Group& g, Node* out) {
+  BitRule none, br;
+  Node* s = nullptr;
+  for (Node* n : g.ins) {
+    if (n->meta.nd == D2) {
+      if (s || n->meta.dt != U8) return none;
+      s = n;
+    } else if (n->kind != Kind::Constant || is_float_dt(n->meta.dt) || n->meta.dt == B8) {
+      return none;
+    }
+  }
+  if (!s || !out || out->meta.dt != U8 || !contains(g.nodes, out)) return none;
+  const std::vector<Node*> all = kernel_order(g);
+  std::set<Node*> in_set(g.ins.begin(), g.ins.end());
+  // the window sums: per node the taps of its three rows (bit 0 left, 1 centre, 2 right)
+  struct Leaf { Node* n; int rows[3], weight, bits; };
+  std::vector<Leaf> leaves;
+  int nbits = 1;  // the centre cell
+  for (Node* n : all) {
+    if (in_set.count(n)) continue;
+    if (is_float_dt(n->meta.dt) || n->meta.dt == B8) return none;
+    if (n->kind == Kind::Constant) {
+      if (is_float_dt(n->cnst.dtype) || n->cnst.dtype == B8) return none;
+      continue;
+    }
+    if (n->meta.nd != D2) return none;
+    if (n->kind == Kind::Convolution || n->kind == Kind::Neighbor) {
+      if (n->prev[0] != s) return none;
+      Leaf f{n, {0, 0, 0}, 0, 0};
+      if (n->kind == Kind::Neighbor) {
+        const int dx = n->coord.arr[0], dy = n->coord.arr[1];
+        if (dx < -1 || dx > 1 || dy < -1 || dy > 1) return none;
+        f.rows[dy + 1] = 1 << (dx + 1);
+        f.weight = 1;
+      } else {
+        if (is_float_dt(n->mask.dtype()) || n->mask.dtype() == B8) return none;
+        const int h0 = n->halo(0), h1 = n->halo(1);
+        if (h0 > 1 || h1 > 1) return none;
+        for (int i1 = -h1; i1 <= h1; i1++)
+          for (int i0 = -h0; i0 <= h0; i0++) {
+            const long long m = variant_as<long long>(n->mask.at(i0 + h0, i1 + h1));
+            if (m < 0 || m > 1) return none;
+            if (m) { f.rows[i1 + 1] |= 1 << (i0 + 1); f.weight++; }
+          }
+      }
+      while ((1 << f.bits) <= f.weight) f.bits++;
+      nbits += f.bits;
+      leaves.push_back(f);
+    } else if (n->pattern() != LOCAL || n->prev.empty() ||
+               !(n->kind == Kind::Cast || n->kind == Kind::Unary || n->kind == Kind::Binary || n->kind == Kind::Conditional)) {
+      return none;
+    }
+  }
+  if (leaves.empty() || nbits > 10) return none;
+  // the group's output for every value of the sums and the centre cell
+  std::string table((size_t)1 << nbits, 'x');
+  std::map<const Node*, Variant> val;
+  auto s32 = [](long long v) { Variant r = variant_zero(S32); r.u.s32 = (int32_t)v; return r; };
+  for (size_t t = 0; t < table.size(); t++) {
+    size_t at = (size_t)nbits;  // the first variable is the highest bit of t
+    bool occurs = true;
+    val.clear();
+    for (const Leaf& f : leaves) {
+      at -= (size_t)f.bits;
+      const int c = (int)((t >> at) & (((size_t)1 << f.bits) - 1));
+      if (c > f.weight) occurs = false;
+      val[f.n] = variant_convert(s32(c), f.n->meta.dt);
+    }
+    if (!occurs) continue;
+    val[s] = variant_convert(s32((long long)(t & 1)), U8);
+    try {
+      for (Node* n : all) {
+        if (val.count(n)) continue;
+        if (n->kind == Kind::Constant) { val[n] = variant_convert(n->cnst, n->meta.dt); continue; }
+        std::vector<Variant> pv;
+        for (Node* p : n->prev) pv.push_back(val.at(p));
+        if (!foldable(n, pv)) return none;
+        val[n] = fold(n, pv);
+      }
+    } catch (const std::exception&) {
+      return none;
+    }
+    const long long o = variant_as<long long>(val.at(out));
+    if (o != 0 && o != 1) return none;
+    table[t] = o ? '1' : '0';
+  }
+  std::vector<std::string> vars;
+  for (size_t i = 0; i < leaves.size(); i++)
+    for (int b = leaves[i].bits - 1; b >= 0; b--) vars.push_back("p" + std::to_string(i) + "[" + std::to_string(b) + "]");
+  vars.push_back("m.c");
+  const std::string e = bool_expr(table, vars, 0);
+  std::ostringstream o;
+  o << "#include \"mapx_dev.hiph\"\nnamespace {\nstruct Rule {\n"
+    << "  template <class V> __device__ static __forceinline__ V f(const mx::BitRow<V>& u, const mx::BitRow<V>& m, const mx::BitRow<V>& d) {\n";
+  for (size_t i = 0; i < leaves.size(); i++)
+    o << "    V p" << i << "[4];\n    mx::win_count<" << leaves[i].rows[0] << ", " << leaves[i].rows[1] << ", "
+      << leaves[i].rows[2] << ">(u, m, d, p" << i << ");\n";
+  o << "    (void)u; (void)m; (void)d;\n    return " << (e == "0" ? "V(0u)" : e == "1" ? "V(~0u)" : e) << ";\n  }\n};\n}  // namespace\n\n";
+  const std::string K = std::to_string(kBitGens);
+  auto kernel = [&](const std::string& tail, const std::string& args, const std::string& body) {
+    o << "extern \"C\" __global__ void __launch_bounds__(256) KRN_NAME" << tail << "(" << args << ") {\n  " << body << "\n}\n";
+  };
+  kernel("_pack", "const mx::u8* in, mx::u32* out, mx::BitGeo g, mx::u32* bad, mx::u32* not_bits, mx::u32 run",
+         "mx::bit_pack(in, out, g, bad, not_bits, run);");
+  for (int rows : kBitRows) {
+    const std::string r = std::to_string(rows);
+    kernel("_step" + r, "const mx::u32* in, mx::u32* out, mx::BitGeo g, int gens, const mx::u32* not_bits, mx::u32 run",
+           "mx::bit_step<Rule, " + r + ", " + K + ">(in, out, g, gens, not_bits, run);");
+  }
+  kernel("_unpack", "const mx::u32* in, mx::u8* out, mx::BitGeo g", "mx::bit_unpack(in, out, g);");
+  std::string src = o.str();
+  br.name = "bit_" + hex_hash(src + dev::header_source());
+  for (size_t pos; (pos = src.find("KRN_NAME")) != std::string::npos;) src.replace(pos, 8, br.name);
+  br.source = src;
+  return br;
 }
 
 }  // namespace mapx

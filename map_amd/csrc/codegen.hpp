@@ -84,6 +84,20 @@ std::vector<Node*> kernel_order(const Group& g);
 // serves them all with its node references rebound by local number.
 std::string kernel_shape_key(const Group& g, const std::vector<Node*>& d2_outs, TileShape tile, bool libm);
 
+// A focal group that is a 3x3 rule on 0/1 rasters: one U8 raster in, one U8
+// raster out that holds 0 or 1 whenever the input does, through 0/1-weighted
+// window sums, neighbours and integer statements of them and constants.
+// `source` is the module of its bit chain (kernels KRN_pack,
+// KRN_step<rows>, KRN_unpack of device/mapx_dev.hiph's bit chains), "" when the
+// group is none.
+struct BitRule {
+  std::string name, source;
+};
+BitRule bit_rule(const Group& g, Node* out);
+constexpr int kBitGens = 8;                      // generations of one step launch
+constexpr int kBitRows[] = {4, 16, 80};          // rows a wavefront of a step kernel owns
+constexpr int kBitShapes = sizeof(kBitRows) / sizeof(kBitRows[0]);
+
 // Default tile shape for a group: VX cells per thread along x so that a
 // wavefront row covers >= 256 contiguous bytes.
 TileShape default_tile(const Group& g);

@@ -927,7 +927,6 @@ void Runtime::radial_task(const Group& g, Eval& e) {
 // the value folded with the neutral, integer PROD the value to the power of
 // the count. Quirk B8 (the reference returns the value itself for SUM) is
 // not reproduced.
-namespace {
 bool foldable(const Node* n, const std::vector<Variant>& pv) {
   switch (n->kind) {
     case Kind::Cast:
@@ -973,6 +972,7 @@ Variant fold(const Node* n, const std::vector<Variant>& pv) {
   return eval_scalar_node(&t);
 }
 
+namespace {
 // acc = OP(acc, v) for `count` taps in the node's C type (the window statements).
 Variant window_fold(const Node* n, const Variant& v) {
   const int dt = n->meta.dt;
@@ -1446,6 +1446,267 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
   }
 }
 
+// ---- bit chains --------------------------------------------------------------------
+// A script that applies one 0/1 rule to a raster many times (the generations
+// of Life) makes a sequence of groups of equal structure, each reading only
+// the raster of the one before. Where nothing else reads or keeps the rasters
+// between, the sequence runs on a bit-packed copy of the first input
+// (device/mapx_dev.hiph, bit chains) and only the last raster is written.
+// The input may hold values above 1, for which the bits are not the raster:
+// the pack kernel reports them (the steps then end at once), the host waits for
+// the sequence and, where a value was reported, runs the groups one by one as
+// if there were no chain.
+
+namespace {
+// One 0/1 raster in and out, and nothing else of a D2 shape: the cheap part of
+// bit_rule's conditions.
+Node* chain_input(const Group& g) {
+  Node* s = nullptr;
+  for (Node* n : g.ins) {
+    if (n->meta.nd != D2) continue;
+    if (s || n->meta.dt != U8) return nullptr;
+    s = n;
+  }
+  return s;
+}
+Node* chain_output(const Group& g) {
+  Node* o = nullptr;
+  for (Node* n : g.outs) {
+    if (n->kind == Kind::Write || n->kind == Kind::Scalar || n->meta.nd != D2 || n->meta.dt != U8 || o) return nullptr;
+    o = n;
+  }
+  if (!o)  // the last group of a script: the node no other reads
+    for (Node* n : g.nodes)
+      if (n->meta.nd == D2 && n->next.empty()) {
+        if (o || n->meta.dt != U8) return nullptr;
+        o = n;
+      }
+  return o && std::find(g.nodes.begin(), g.nodes.end(), o) != g.nodes.end() ? o : nullptr;
+}
+// What bit_rule depends on, as bytes: the group's nodes in the kernel's local
+// numbering with their constants. "" for a group that reads a D0 value which is
+// no constant. Groups of equal keys are one rule.
+std::string rule_key(const Group& g, const Node* out) {
+  const std::vector<Node*> all = kernel_order(g);
+  std::string k;
+  auto put = [&](int v) { k.append((const char*)&v, sizeof v); };
+  auto put_value = [&](const Variant& v) {
+    const uint64_t b = variant_bits(v);
+    put(v.dtype);
+    k.append((const char*)&b, sizeof b);
+  };
+  for (size_t i = 0; i < all.size(); i++) {
+    const Node* n = all[i];
+    put(n->meta.nd);
+    put(n->meta.dt);
+    put(n == out);
+    if (i < g.ins.size()) {  // kernel_order: inputs first
+      if (n->meta.nd == D2) continue;
+      if (n->kind != Kind::Constant) return "";
+      put_value(n->cnst);
+      continue;
+    }
+    put((int)n->kind);
+    put(n->op);
+    if (n->kind == Kind::Constant) put_value(n->cnst);
+    if (n->kind == Kind::Neighbor) { put(n->coord.arr[0]); put(n->coord.arr[1]); }
+    if (n->kind == Kind::Convolution) {
+      put(n->mask.ds.arr[0]);
+      put(n->mask.ds.arr[1]);
+      for (const Variant& v : n->mask.v) put_value(v);
+    }
+    put((int)n->prev.size());
+    for (const Node* p : n->prev) {
+      size_t j = 0;
+      while (j < all.size() && all[j] != p) j++;
+      put((int)j);
+    }
+  }
+  return k;
+}
+struct BitGeoHost { int W, H, WD, BS0, BS1, NB0; };  // mx::BitGeo
+// threads of the pack and unpack kernels: 16 cells x 4 rows each
+long bit_spots(const Meta& m) { return 2L * ((m.ds.arr[0] + 31) / 32) * ((m.ds.arr[1] + 3L) / 4); }
+constexpr size_t kBitFlags = 1024;                   // chains of one level that run together
+}  // namespace
+
+void Runtime::find_bit_chains(Plan& plan) {
+  std::unordered_map<Node*, std::vector<const Group*>> readers;
+  for (auto& g : plan.groups)
+    for (Node* n : g->ins)
+      if (n->meta.nd == D2) readers[n].push_back(g.get());
+  std::unordered_set<const Group*> taken;
+  for (auto& gp : plan.groups) {  // in dependency order: a chain is met at its first group
+    const Group* g = gp.get();
+    if (taken.count(g) || !pattern_is(g->pat, FOCAL) || pattern_is(g->pat, ZONAL)) continue;
+    BitChain c;
+    c.in = chain_input(*g);
+    Node* o = chain_output(*g);
+    if (!c.in || !o || c.in->meta.bs.arr[0] % 32 || !dim2_eq(o->meta.ds, c.in->meta.ds) ||
+        !dim2_eq(o->meta.bs, c.in->meta.bs) || bit_spots(o->meta) >= (1L << 31) - 256)
+      continue;
+    const std::string key = rule_key(*g, o);
+    if (key.empty()) continue;
+    for (;;) {
+      c.groups.push_back(g);
+      c.out.push_back(o);
+      auto r = readers.find(o);
+      if (r == readers.end() || r->second.size() != 1) break;
+      const Group* h = r->second[0];
+      Node* p = chain_output(*h);
+      if (taken.count(h) || !p || chain_input(*h) != o || rule_key(*h, p) != key) break;
+      g = h;
+      o = p;
+    }
+    if (c.groups.size() < kBitChain) continue;
+    for (const Group* h : c.groups) taken.insert(h);
+    auto known = bit_kernels_.find(key);
+    if (known == bit_kernels_.end()) {
+      if (bit_kernels_.size() >= 4096) bit_kernels_.clear();  // bounded; plans keep theirs
+      HostTimer ht(cnt.ms_codegen);
+      auto k = std::make_shared<BitKernels>();
+      const BitRule br = bit_rule(*c.groups[0], c.out[0]);
+      if (!br.source.empty()) {
+        k->name = br.name;
+        k->pack = dev::function(br.source, br.name + "_pack").fn;
+        for (int i = 0; i < kBitShapes; i++)
+          k->step[i] = dev::function(br.source, br.name + "_step" + std::to_string(kBitRows[i])).fn;
+        k->unpack = dev::function(br.source, br.name + "_unpack").fn;
+        kernel_src_[br.name] = br.source;
+        cnt.compiles++;
+      }
+      known = bit_kernels_.emplace(key, std::move(k)).first;
+    }
+    if (!known->second->unpack) continue;  // no bit rule
+    c.k = known->second;
+    for (size_t i = 0; i < c.groups.size(); i++) plan.chain_at[c.groups[i]] = {plan.chains.size(), i};
+    plan.chains.push_back(std::move(c));
+  }
+}
+
+// Groups first..first+n-1 of a chain: the last one's raster from the first
+// one's input. Two bit rasters (an eighth of a U8 one each) come from the
+// store for the launches.
+void Runtime::launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t slot) {
+  HostTimer ht(cnt.ms_launch);
+  Node* in = first ? c.out[first - 1] : c.in;
+  Node* on = c.out[first + n - 1];
+  ensure_input(in);
+  const Meta& m = on->meta;
+  void* out = store.alloc(rasterBytes(m));
+  resident_[on] = out;
+  BitGeoHost g{m.ds.arr[0], m.ds.arr[1], (m.ds.arr[0] + 31) / 32, m.bs.arr[0], m.bs.arr[1], m.nb(0)};
+  struct Bits {  // given back in stream order, also when a launch fails
+    Store& st;
+    void* p;
+    Bits(Store& s, size_t bytes) : st(s), p(s.alloc(bytes)) {}
+    ~Bits() { st.release(p); }
+  };
+  const size_t bytes = (size_t)g.WD * 4 * (size_t)g.H;
+  Bits bits_a(store, bytes), bits_b(store, bytes);
+  void *a = bits_a.p, *b = bits_b.p;
+  void* src = residentPtr(in);
+  auto launch = [&](void* fn, const char* tail, unsigned grid, std::vector<std::pair<void*, size_t>> args) {
+    std::vector<void*> p;
+    std::vector<size_t> z;
+    for (auto& x : args) { p.push_back(x.first); z.push_back(x.second); }
+    dev::Function f;
+    f.fn = fn;
+    f.name = c.k->name + tail;
+    dev::launch(f, grid, 256, p.data(), z.data(), (int)p.size());
+    cnt.launches++;
+  };
+  const long spots = bit_spots(m);
+  const unsigned pgrid = (unsigned)((spots + 255) / 256);
+  void *bad = bit_flags_ + slot, *not_bits = bit_runs_ + slot;
+  uint32_t run = ++bit_run_;
+  launch(c.k->pack, "_pack", pgrid, {{&src, 8}, {&a, 8}, {&g, sizeof g}, {&bad, 8}, {&not_bits, 8}, {&run, 4}});
+  // Rows a wavefront owns: it computes 2 * kBitGens more, and the SIMD with the
+  // most wavefronts decides the time of a launch.
+  const long nsx = (g.WD + 61) / 62, simds = 4L * std::max(1, dev::num_cus());
+  int shape = 0;
+  long waves = 0, best = 0;
+  for (int i = 0; i < kBitShapes; i++) {
+    const long w = nsx * ((g.H + kBitRows[i] - 1L) / kBitRows[i]);
+    const long cost = ((w + simds - 1) / simds) * (kBitRows[i] + 2 * kBitGens);
+    if (i == 0 || cost < best) { best = cost; waves = w; shape = i; }
+  }
+  const std::string step = "_step" + std::to_string(kBitRows[shape]);
+  for (size_t done = 0; done < n; done += kBitGens) {
+    int gens = (int)std::min<size_t>(kBitGens, n - done);
+    launch(c.k->step[shape], step.c_str(), (unsigned)((waves + 3) / 4), 
+           {{&a, 8}, {&b, 8}, {&g, sizeof g}, {&gens, 4}, {&not_bits, 8}, {&run, 4}});
+    std::swap(a, b);
+  }
+  launch(c.k->unpack, "_unpack", pgrid, {{&a, 8}, {&out, 8}, {&g, sizeof g}});
+}
+
+// Measured, one evaluation of n generations, chain against groups: 256^2 cells
+// 39 / 35 us (n = 4) and 47 / 56 (8); 1024^2 40 / 38 (4) and 47 / 60 (8); 4096^2
+// 43 / 40 (2) and 45 / 53 (3); 16384^2 154 / 343 (2). A group costs 5 us and
+// 0.6 ns per 1000 cells; a chain 17 us more than one launch and 0.4 ns per
+// 1000 cells for its pack and unpack, and little per generation.
+bool Runtime::bit_chain_pays(size_t n, const Meta& m) {
+  const double cells = (double)m.ds.arr[0] * m.ds.arr[1];
+  return (double)n * (3.5 + 0.57e-6 * cells) > 20.0 + 0.37e-6 * cells;
+}
+
+// Runs the chains that begin at this level (the rest of their groups are on
+// later ones) and marks the groups they computed in `e.done`.
+void Runtime::run_bit_chains(Eval& e, size_t level) {
+  if (opt.form == FORM_PLAIN || opt.tile.TX > 0 || e.plan->chains.empty()) return;
+  struct Run { const BitChain* c; size_t first, n; };
+  std::vector<Run> runs;
+  for (const Group* g : e.levels[level]) {
+    auto it = e.plan->chain_at.find(g);
+    if (it == e.plan->chain_at.end() || e.not_bits.count(g)) continue;
+    const BitChain& c = e.plan->chains[it->second.first];
+    // from here as far as nobody keeps or asks for a raster between
+    size_t i = it->second.second, n = 0;
+    while (i + n < c.groups.size()) {
+      const Group& h = *c.groups[i + n];
+      if (e.done.count(&h)) break;
+      bool zonal = false;
+      const std::vector<Node*> outs = kernel_outputs(h, e.tsorted, zonal);
+      if (outs.size() != 1 || outs[0] != c.out[i + n]) break;
+      n++;
+      if (ext_refs(outs[0]) > 0 || e.tset.count(outs[0])) break;
+    }
+    if (n >= kBitChain && bit_chain_pays(n, c.out[i]->meta)) runs.push_back({&c, i, n});
+  }
+  if (runs.empty()) return;
+  PauseRecording pause;
+  if (!bit_runs_) {
+    if (!bit_flags_) bit_flags_ = (uint32_t*)dev::malloc_host(kBitFlags * sizeof(uint32_t));
+    std::memset(bit_flags_, 0, kBitFlags * sizeof(uint32_t));
+    void* d = alloc_outside_store(store, kBitFlags * sizeof(uint32_t));
+    dev::h2d(d, bit_flags_, kBitFlags * sizeof(uint32_t));  // run numbers start at 1
+    dev::sync();
+    bit_runs_ = (uint32_t*)d;
+  }
+  volatile uint32_t* bad = bit_flags_;
+  for (size_t r0 = 0; r0 < runs.size(); r0 += kBitFlags) {
+    const size_t r1 = std::min(runs.size(), r0 + kBitFlags);
+    for (size_t r = r0; r < r1; r++) {
+      bad[r - r0] = 0;
+      launch_bit_chain(*runs[r].c, runs[r].first, runs[r].n, r - r0);
+    }
+    dev::sync();
+    for (size_t r = r0; r < r1; r++) {
+      const Run& x = runs[r];
+      if (bad[r - r0]) {  // not a 0/1 raster
+        Node* on = x.c->out[x.first + x.n - 1];
+        store.release(resident_.at(on));
+        resident_.erase(on);
+        for (size_t i = 0; i < x.n; i++) e.not_bits.insert(x.c->groups[x.first + i]);
+      } else {
+        cnt.groups += (long)x.n;
+        for (size_t i = 0; i < x.n; i++) e.done.insert(x.c->groups[x.first + i]);
+      }
+    }
+  }
+}
+
 // Runs one level of each evaluation: host scalar groups at once, kernels of
 // all evaluations batched by kernel.
 void Runtime::run_levels(const std::vector<std::pair<Eval*, size_t>>& work, std::vector<Readback>* async) {
@@ -1457,7 +1718,8 @@ void Runtime::run_levels(const std::vector<std::pair<Eval*, size_t>>& work, std:
   std::vector<std::pair<Eval*, const Group*>> groups;
   groups.reserve(n);
   for (auto& w : work)
-    for (const Group* gp : w.first->levels[w.second]) groups.push_back({w.first, gp});
+    for (const Group* gp : w.first->levels[w.second])
+      if (!w.first->done.count(gp)) groups.push_back({w.first, gp});
   const bool whole = dev::recording() || opt.form == FORM_PLAIN;
   size_t i = 0;
   for (size_t g0 = 0, g1 = 0; g0 < groups.size(); g0 = g1) {
@@ -1573,6 +1835,7 @@ void Runtime::eval_plan(Eval& e) {
       HostTimer ht(cnt.ms_fuse);
       pl->groups = Fuser(fo).fuse(e.list);
     }
+    if (!serving()) find_bit_chains(*pl);
     pit = plans_.emplace(pkey, std::move(pl)).first;
   }
   e.plan = pit->second;
@@ -1689,6 +1952,7 @@ void Runtime::evaluate(const std::vector<Node*>& targets) {
       const bool big = e.levels[l].size() >= (size_t)kBigLevel;
       const bool rec = dev::recording();
       if (big && rec) dev::record_flush();
+      run_bit_chains(e, l);
       run_levels({{&e, l}}, &pend);
       if (big && rec) dev::record_begin();
       eval_release(e, l);
@@ -1762,6 +2026,10 @@ std::string Runtime::plan(const std::vector<Node*>& targets_in) {
     if (Node* sn = spread_node(*g)) {  // precompiled walk kernels (spread.hip)
       j << ", \"spread\": {\"reduction\": " << sn->op << "}}";
       continue;
+    }
+    if (pattern_is(g->pat, FOCAL) && chain_input(*g) && chain_output(*g)) {
+      const BitRule br = bit_rule(*g, chain_output(*g));
+      if (!br.source.empty()) j << ", \"bit_rule\": \"" << esc(br.source) << "\"";
     }
     if (!host_group(*g)) {
       std::vector<Node*> outs = d2_outputs(*g, tsorted), kouts;

@@ -173,6 +173,8 @@ class Runtime {
     std::vector<std::vector<const Group*>> levels;
     std::unordered_map<Node*, int> uses;
     std::unordered_set<Node*> tset;
+    std::unordered_set<const Group*> done;      // groups a bit chain has computed
+    std::unordered_set<const Group*> not_bits;  // groups of a chain whose input was not 0/1
     // kernels fixed at planning time (requests of the server run later)
     std::unordered_map<const Group*, std::pair<std::vector<Node*>, KernelEntry*>> kern;
   };
@@ -183,6 +185,7 @@ class Runtime {
   void eval_finish(Eval& e);
   std::vector<Node*> kernel_outputs(const Group& g, const std::vector<Node*>& targets, bool& has_zonal);
   void run_levels(const std::vector<std::pair<Eval*, size_t>>& work, std::vector<Readback>* async);
+  static constexpr size_t kBitChain = 2;  // groups a bit chain replaces at least (bit_chain_pays)
   static constexpr int kBigLevel = 64;    // levels of at least this many groups run unrecorded
   static constexpr int kSubBatch = 512;   // groups prepared and launched together when unrecorded
   static constexpr int kFirstSubBatch = 64;  // the first of them
@@ -218,8 +221,30 @@ class Runtime {
     void* fin = nullptr;
     int occ = 0;  // resident work-groups per CU
   };
+  // A sequence of groups that apply one bit rule (codegen's bit_rule), each to
+  // the raster of the one before and to nothing else.
+  struct BitKernels {
+    std::string name;
+    void *pack = nullptr, *step[kBitShapes] = {}, *unpack = nullptr;
+  };
+  struct BitChain {
+    std::vector<const Group*> groups;
+    std::vector<Node*> out;  // the raster of each group
+    Node* in = nullptr;      // the first group's input
+    std::shared_ptr<const BitKernels> k;
+  };
+  std::unordered_map<std::string, std::shared_ptr<BitKernels>> bit_kernels_;  // by rule; no kernels: no bit rule
+  void find_bit_chains(Plan& plan);
+  void run_bit_chains(Eval& e, size_t level);
+  void launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t slot);
+  static bool bit_chain_pays(size_t n, const Meta& m);
+  uint32_t* bit_flags_ = nullptr;  // pinned words the pack kernels report to
+  uint32_t* bit_runs_ = nullptr;   // and words in HBM that end the steps of a run that is no 0/1 raster
+  uint32_t bit_run_ = 0;           // number of the last run
   struct Plan {
     std::vector<std::unique_ptr<Group>> groups;
+    std::vector<BitChain> chains;
+    std::unordered_map<const Group*, std::pair<size_t, size_t>> chain_at;  // group -> (chain, place in it)
     std::map<std::pair<const Group*, std::vector<Node*>>, KernelEntry> kernels;
   };
   std::string plan_key(const std::vector<Node*>& list, const std::vector<Node*>& targets) const;
@@ -292,5 +317,9 @@ class Runtime {
 // Host evaluation of a D0 node from its (D0) prevs, with C semantics in the
 // node types (ScalarTask, runtime/task/ScalarTask.cpp:69-193).
 Variant eval_scalar_node(const Node* n);
+// A statement on known operand values: whether its host evaluation gives the
+// device's bits, and the value (constant-raster prediction, bit rules).
+bool foldable(const Node* n, const std::vector<Variant>& pv);
+Variant fold(const Node* n, const std::vector<Variant>& pv);
 
 }  // namespace mapx
