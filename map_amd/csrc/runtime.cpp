@@ -1114,9 +1114,9 @@ Node* Runtime::spread_node(const Group& g) {
 }
 
 // A spreading group is its SpreadScan node alone: the accumulation of a
-// resident raster along the resident direction raster (spread.hip: tiles in
-// LDS that also count and list the walk sources, then the walks), with a count
-// word per cell and the source list taken from the store for the launches.
+// resident raster along the resident direction raster (spread.hip: visits to
+// tiles from a queue), with the finished bits and the queue taken from the store
+// for the launches.
 void Runtime::spread_task(const Group& g, Eval& e) {
   Node* n = spread_node(g);
   if (g.nodes.size() != 1) fail("spread scan fused with other nodes");
@@ -1127,12 +1127,13 @@ void Runtime::spread_task(const Group& g, Eval& e) {
   const Meta& m = n->meta;
   void* out = store.alloc(rasterBytes(m));
   resident_[n] = out;
-  const size_t cells = (size_t)m.bs.arr[0] * m.bs.arr[1] * m.nb(0) * m.nb(1);
-  void* counts = store.alloc(cells * 8 + 8);  // a status word per cell, then the list of walk sources
+  // per 64x64 tile: 17 bits per cell, a notification word and a queue entry; the queues' counters
+  const size_t tiles = (size_t)((m.ds.arr[0] + 63) / 64) * ((m.ds.arr[1] + 63) / 64);
+  void* scratch = store.alloc(tiles * (8192 + 512 + 8) + 64 * 256 + 64 * 4);
   PauseRecording pause;
-  cnt.launches += spread::run(out, residentPtr(n->prev[0]), residentPtr(n->prev[1]), counts, m.dt, m.bs.arr[0],
+  cnt.launches += spread::run(out, residentPtr(n->prev[0]), residentPtr(n->prev[1]), scratch, m.dt, m.bs.arr[0],
                               m.bs.arr[1], m.nb(0), m.nb(1), m.ds.arr[0], m.ds.arr[1], dev::stream());
-  store.release(counts);  // reused in stream order, after the walks
+  store.release(scratch);  // reused in stream order, after the visits
 }
 
 bool Runtime::prepare_task(const Group& g, Eval& e, Task& t) {
