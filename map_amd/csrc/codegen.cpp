@@ -243,6 +243,12 @@ TileShape default_tile(const Group& g) {
     if (n->meta.nd == D2 && (std::find(g.outs.begin(), g.outs.end(), n) != g.outs.end() || n->next.empty()))
       minsz = std::min(minsz, sizeof_dt(n->meta.dt));
   if (minsz == 8) minsz = 4;
+  // windows of 4-byte cells in LDS: 16 bytes a lane, lanes side by side. Eight
+  // cells a lane (a 1-byte raster beside them) put a wavefront's reads on half of
+  // the banks and take twice the registers: slope and statistics over U8 zones,
+  // 254M cells, 1387 us with 8 cells and 1103 with 4.
+  for (Node* n : g.nodes)
+    if (n->pattern() == FOCAL && sizeof_dt(n->prev[0]->meta.dt) >= 4) minsz = std::max(minsz, 4);
   TileShape t;
   // 64 threads per tile row, each moving one vector of the narrowest type:
   // 8 cells of 1-byte types, 4 cells of 2- and 4-byte types, 2 of 8-byte types
@@ -304,6 +310,13 @@ std::string kernel_shape_key(const Group& g, const std::vector<Node*>& d2_outs, 
     k << (it == local.end() ? -1 : it->second) << ",";
   }
   return k.str();
+}
+
+int fold_groups(const KernelSpec& ks) {
+  int most = 1;
+  for (const ZonalOut& z : ks.zouts)
+    if (z.node->kind == Kind::ZonalStats) most = std::max(most, z.nzones);
+  return (most + 15) / 16;
 }
 
 KernelSpec generate_kernel(const Group& g, const std::vector<Node*>& d2_outs, TileShape tile, bool libm) {
@@ -954,41 +967,36 @@ KernelSpec generate_kernel(const Group& g, const std::vector<Node*>& d2_outs, Ti
     << ", (MX_NARROW != 0)>(a0, L0, tasks, starts, ntasks, nchunks, queue, zpart, acc, sm, &slot);\n";
   s << "}\n";
 
-  // fold kernel: folds partial records in index order. Work-group (f, t) folds
-  // slice f of F of task t's records [base, base+n) of `src` into record
-  // t*F + f of `dst`: task t's chunks (tasks: from the table; stride == 0: one
-  // task of n_single chunks) or, with stride > 0, records [t*stride, (t+1)*stride).
+  // fold kernel: work-group (f, g) of task t folds slice f of the task's records
+  // in `src` (its chunks, from the table or one task of n_single; with stride > 0
+  // the slices' records of the first pass, at t * stride) into record t*F + f of
+  // `dst`, for the 16 zones of group g. The slices depend on the task's number of
+  // chunks alone, so a task's sums are the same alone and in a batch.
   if (!zonal.empty()) {
     s << "\nextern \"C\" __global__ void __launch_bounds__(256) " << ks.fin_name
       << "(const char* src, char* dst, const mx::TaskRec<P::Args>* tasks, const int* starts, int n_single, int stride, int F) {\n";
     s << "  __shared__ mx::u64 red_scratch[4];\n";
-    s << "  const int t = blockIdx.y, f = blockIdx.x;\n";
+    s << "  const int t = blockIdx.y, f = blockIdx.x / " << fold_groups(ks) << ", g = blockIdx.x % " << fold_groups(ks) << ";\n";
     s << "  int base = 0, n = n_single;\n";
     s << "  if (tasks) { base = tasks[t].L.part0; n = starts[t + 1] - starts[t]; }\n";
-    s << "  else if (stride > 0) { base = t * stride; n = stride; }\n";
-    s << "  const int b0 = base + (int)((long long)n * f / F), b1 = base + (int)((long long)n * (f + 1) / F);\n";
+    s << "  int slices = mx::fold_slices(n);\n";
+    s << "  if (stride > 0) { base = t * stride; n = slices; slices = 1; }\n";
+    s << "  if (f >= slices) return;\n";
+    s << "  const int b0 = base + (int)((long long)n * f / slices), b1 = base + (int)((long long)n * (f + 1) / slices);\n";
     s << "  char* out = dst + (size_t)(t * F + f) * " << part_bytes << "u;\n";
     for (size_t j = 0; j < ks.zouts.size(); j++) {
       const ZonalOut& z = ks.zouts[j];
       if (z.node->kind == Kind::ZonalReduc) {
         std::string A = CT(z.acc_dt);
-        s << "  {\n    " << A << " r = " << lit(reduction_neutral(z.red, z.acc_dt)) << ";\n";
+        s << "  if (g == 0) {\n    " << A << " r = " << lit(reduction_neutral(z.red, z.acc_dt)) << ";\n";
         s << "    for (int p = b0 + threadIdx.x; p < b1; p += 256) r = " << red_op(z.red) << "::f(r, *(const " << A
           << "*)(src + (size_t)p * " << part_bytes << "u + " << part_off[j] << "));\n";
         s << "    mx::block_reduce_store<" << red_op(z.red) << ", " << A << ">(r, (" << A << "*)(out + " << part_off[j]
           << "), (" << A << "*)red_scratch);\n  }\n";
       } else {
         std::string T = CT(z.dt);
-        std::string M = std::string("mx::MM<") + T + ">::t";
-        s << "  for (int zi = threadIdx.x; zi < " << z.nzones << "; zi += 256) {\n";
-        s << "    double sum = 0.0; " << M << " mn = mx::mm_highest<" << T << ">(), mxv = mx::mm_lowest<" << T
-          << ">(); mx::u32 cnt = 0u;\n";
-        s << "    for (int p = b0; p < b1; p++) {\n";
-        s << "      const mx::ZonePart<" << T << ">& q = ((const mx::ZonePart<" << T << ">*)(src + (size_t)p * "
-          << part_bytes << "u + " << part_off[j] << "))[zi];\n";
-        s << "      sum += q.sum; mn = mx::OpMin::f(mn, q.mn); mxv = mx::OpMax::f(mxv, q.mx); cnt += q.cnt;\n    }\n";
-        s << "    mx::ZonePart<" << T << "> r; r.sum = sum; r.mn = mn; r.mx = mxv; r.cnt = cnt; r.pad = 0u;\n";
-        s << "    ((mx::ZonePart<" << T << ">*)(out + " << part_off[j] << "))[zi] = r;\n  }\n";
+        s << "  mx::zone_fold<" << T << ", " << z.nzones << ">(src + " << part_off[j] << ", " << part_bytes
+          << "u, b0, b1, g, (mx::ZonePart<" << T << ">*)(out + " << part_off[j] << "));\n";
       }
     }
     s << "}\n";
