@@ -104,6 +104,8 @@ def check(t, v, z, nz):
     cnt = np.bincount(zz, minlength=nz)
     assert np.array_equal(t["count"], cnt)
     assert np.array_equal(t["sum"], np.bincount(zz, weights=v64, minlength=nz))
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(t["mean"], np.where(cnt > 0, t["sum"] / np.maximum(cnt, 1), np.nan), equal_nan=True)
     mn, mx = np.full(nz, np.inf), np.full(nz, -np.inf)
     np.minimum.at(mn, zz, v64)
     np.maximum.at(mx, zz, v64)
