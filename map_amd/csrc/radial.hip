@@ -20,7 +20,10 @@
 // every raster), from which the next band reads its starting column.
 //
 // What bounds it: the chain of columns. A column is 2 rows x 20 instructions in
-// a wavefront, and a launch of a large raster has about one wavefront per SIMD.
+// a wavefront, about 260 cycles of dependent ones, and a launch of a large raster
+// has about one wavefront per SIMD. (One launch for all bands, with wavefronts
+// that wait for the row before theirs, took as long: each hand-over costs what
+// 16 columns do.)
 // The division of the interpolation weight, d1/d0, is by a number that all rows
 // of a column share: q = d1 * (1/d0), then q + (d1 - q d0) * (1/d0) with fused
 // multiply-adds is the correctly rounded quotient (Markstein, IBM Journal of
@@ -30,8 +33,10 @@
 // apart, and along x, where the rows are a block row apart, a row's K cells move as vectors.
 // (Cell by cell, with a step through the blocks for each, the addresses took more instructions
 // than the columns; that path is left for block sides that K does not divide.)
-// 16384^2 F32 from the centre: 2.5 ms, 20 us a band (a work-group of 256 rows exchanging
-// columns through LDS with a barrier, cells moved one by one: 4.8 ms).
+// 16384^2 F32 from the centre: 2.4 ms, 18.7 us a band (a work-group of 256 rows exchanging
+// columns through LDS with a barrier, cells moved one by one: 4.8 ms; a branch around the
+// operation for inputs that are not finite, and the diagonal's selection in every band:
+// 20 us a band).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -160,7 +165,8 @@ template <class T> struct Row {
 };
 
 // R of row r at column c: cf = (T)c, y = 1 / cf, a = R of row r, nb = R of row r - 1 at column c - 1.
-template <class T, int OP, bool QUICK>
+// (DIAG: the row may be on the diagonal.)
+template <class T, int OP, bool QUICK, bool DIAG>
 __device__ __forceinline__ T radial_step(const Row<T>& row, int c, T cf, T y, T a, T nb, T x) {
   // linear_interpolation's weight (runtime/skeleton/util.cpp:564; its float literals are exact here)
   T q;
@@ -172,14 +178,16 @@ __device__ __forceinline__ T radial_step(const Row<T>& row, int c, T cf, T y, T 
   }
   const T w = q * (cf - (T)1) - row.m1;
   const T mix = a * w + nb * ((T)1 - w);  // a*w + b*(1-w)
-  T base = row.r == c ? nb : mix;
+  T base = DIAG && row.r == c ? nb : mix;
   base = row.r == 0 ? a : base;
-  return __builtin_isfinite(x) ? combine<OP>(base, x) : base;
+  const T both = combine<OP>(base, x);  // not under the condition: the instruction would get a branch
+  return __builtin_isfinite(x) ? both : base;
 }
 
-// The columns of a band, position by position (FULL: all of them are in it). va, vb: the rows'
+// The columns of a band, position by position (FULL: all of them are in it; DIAG: some row
+// may be on the diagonal). va, vb: the rows'
 // inputs; the owned row's results replace vb.
-template <class T, int OP, int K, bool QUICK, bool FULL>
+template <class T, int OP, int K, bool QUICK, bool FULL, bool DIAG>
 __device__ __forceinline__ void columns(const Oct& O, const Row<T>& ra, const Row<T>& rb, T pa, T pb, const T (&va)[K], T (&vb)[K]) {
   // lane p: column cb + p and its reciprocal
   const T cl = (T)(O.cb + (int)(threadIdx.x & 63)), yl = (T)1 / cl;
@@ -188,8 +196,8 @@ __device__ __forceinline__ void columns(const Oct& O, const Row<T>& ra, const Ro
     if (!FULL && (p < O.p0 || p >= O.p1)) continue;  // uniform
     const T cf = lane_read(cl, p), y = lane_read(yl, p);
     const T na = lane_prev(pa), nb = lane_prev(pb, lane_read(pa, 63));
-    pa = radial_step<T, OP, QUICK>(ra, O.cb + p, cf, y, pa, na, va[p]);
-    pb = radial_step<T, OP, QUICK>(rb, O.cb + p, cf, y, pb, nb, vb[p]);
+    pa = radial_step<T, OP, QUICK, DIAG>(ra, O.cb + p, cf, y, pa, na, va[p]);
+    pb = radial_step<T, OP, QUICK, DIAG>(rb, O.cb + p, cf, y, pb, nb, vb[p]);
     vb[p] = pb;
   }
 }
@@ -264,8 +272,9 @@ __global__ void __launch_bounds__(NT) k_radial(const T* __restrict__ in, T* __re
       for (int p = 0; p < K; p++) { va[p] = a[(K - 1 - p) / V].v[(K - 1 - p) % V]; vb[p] = b[(K - 1 - p) / V].v[(K - 1 - p) % V]; }
     }
   }
-  if (full) columns<T, OP, K, QUICK, true>(O, ra, rb, pa, pb, va, vb);
-  else columns<T, OP, K, QUICK, false>(O, ra, rb, pa, pb, va, vb);
+  if (full && r0 + 2 * OWN - 1 < O.cb) columns<T, OP, K, QUICK, true, false>(O, ra, rb, pa, pb, va, vb);
+  else if (full) columns<T, OP, K, QUICK, true, true>(O, ra, rb, pa, pb, va, vb);
+  else columns<T, OP, K, QUICK, false, true>(O, ra, rb, pa, pb, va, vb);
   // the owned rows' results of the band
   if (rb.r > O.L1) return;
   const bool whole = full && r0 + 2 * OWN - 1 <= O.cb;  // uniform: no cell of the band outside the octant
