@@ -848,10 +848,9 @@ uint32_t morton2(uint32_t x, uint32_t y) {
 constexpr int kZonalChunkCells = 65536, kZonalChunks = 256;
 // Tiles per chunk of other groups: consecutive tiles of a block run on one
 // work-group (halo rows shared with the previous tile are still in L2), at
-// most kChunkTiles, fewer when the launch would otherwise leave work-groups
-// idle or unevenly loaded (at least eight chunks per work-group of the grid: a
-// 5x5 convolution of 128 rasters, 254M cells, took 708 us with two and 587 with
-// eight; a task's first chunk costs a lookup, so not more).
+// most kChunkTiles. Batches, whose tasks differ, take chunks from the queue: at
+// least eight per work-group of the grid (a 5x5 convolution of 128 rasters, 254M
+// cells, took 708 us with two and 587 with eight).
 constexpr int kChunkTiles = 16;
 int adaptive_chunk(long tiles_total, int grid_max) {
   const long per = tiles_total / (8L * std::max(1, grid_max));
@@ -883,6 +882,24 @@ struct Runtime::Task {
     auto chunks = [&](bool l0, bool l1) { return (tiles(l0, l1) + L.CH - 1) / L.CH; };
     L.C00 = chunks(false, false); L.C10 = chunks(true, false); L.C01 = chunks(false, true); L.C11 = chunks(true, true);
     nchunks = first_chunk(L.NB0 * L.NB1);
+  }
+  // One task in a static split. Few tiles per work-group: the tiles per chunk for
+  // which the work-groups' turns cost least, a turn being its tiles and a tenth of
+  // one for the chunk itself (hillshade 4096^2, 4 tiles per work-group: 76.1 us in
+  // chunks of 4, 78.8 of 2, 80.7 of 1). Many: two chunks per work-group or more (a
+  // work-group's tiles in one chunk, a block's rows apart, load the same HBM
+  // channels as its neighbours': Life by groups 0.118 ms in chunks of 5, 0.129 of 8).
+  void chunking_static(int grid_max) {
+    const long tiles = this->tiles();
+    if (tiles >= 8L * grid_max) return chunking((int)std::min<long>(kChunkTiles, tiles / (2L * grid_max)));
+    int best = 1;
+    long least = 0;
+    for (int ch = 1; ch <= 8; ch++) {
+      chunking(ch);
+      const long turns = (nchunks + grid_max - 1) / grid_max, cost = turns * (10L * ch + 1);
+      if (ch == 1 || cost < least) { best = ch; least = cost; }
+    }
+    chunking(best);
   }
   // chunks before block b (block rows in order)
   int first_chunk(int b) const {
@@ -1426,7 +1443,8 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
   if (batch.size() == 1) {
     Task* t = batch[0];
     const bool q = opt.queue == 1;
-    t->chunking(opt.chunk_tiles > 0 ? opt.chunk_tiles : adaptive_chunk(t->tiles(), gmax));
+    if (opt.chunk_tiles > 0 || zonal) t->chunking(opt.chunk_tiles);
+    else t->chunking_static(gmax);
     void* parts = zonal ? store.alloc((size_t)t->nchunks * ks.part_bytes) : nullptr;
     launch(t->args, t->L, nul, nul, 1, t->nchunks, q ? queue() : nul, parts, grid_for(t->nchunks));
     if (zonal) {
