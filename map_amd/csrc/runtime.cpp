@@ -839,13 +839,17 @@ uint32_t morton2(uint32_t x, uint32_t y) {
   return spread(x) | (spread(y) << 1);
 }
 
-// Cells per chunk of a zonal group (one partial record per chunk): a 256th of
-// the raster, so that a raster evaluated alone has a chunk for every CU, at
-// least a tile and at most 65536, where a large raster has chunks enough and
-// more would only add records to fold. Decided by the raster's size alone, so
-// sums do not depend on what else is launched. With 65536 throughout, the
-// statistics of one raster of 1.2M cells ran on 16 work-groups: 201 us, now 21.
-constexpr int kZonalChunkCells = 65536, kZonalChunks = 256;
+// Cells per chunk of a zonal group (one partial record per chunk): a part of the
+// raster, so that a raster evaluated alone has chunks enough for every CU, at
+// least a tile and at most 65536 cells, where more chunks would only add records
+// to fold. Decided by the raster and the kernel alone, so sums do not depend on
+// what else is launched. Groups with windows compute long per tile and want
+// several chunks per work-group: hillshade with statistics of 4096^2 took 240 us
+// in chunks of 65536 cells, 106 in a 512th, 91 in a 2048th; of 8000x7000 324, 329
+// and 264. Cell-wise groups wait for HBM, and long runs read it better: an overlay
+// of 8191x6001 took 175 us in a 512th and 186 in a 2048th, of 3000x2500 75 in
+// chunks of 65536 cells and 30 in a 512th.
+constexpr int kZonalChunkCells = 65536, kZonalChunksFocal = 2048, kZonalChunksLocal = 512;
 // Tiles per chunk of other groups: consecutive tiles of a block run on one
 // work-group (halo rows shared with the previous tile are still in L2), at
 // most kChunkTiles. Batches, whose tasks differ, take chunks from the queue: at
@@ -1233,7 +1237,8 @@ bool Runtime::prepare_task(const Group& g, Eval& e, Task& t) {
   const int BS0 = gm.bs.arr[0], BS1 = gm.bs.arr[1], NB0 = gm.nb(0), NB1 = gm.nb(1);
   t.L = HostLaunch{BS0, BS1, NB0, NB1, gm.ds.arr[0], gm.ds.arr[1], -1, 1, 1, 1, 1, 1, 0};
   if (!ks.zouts.empty()) {
-    const long cells = std::min<long>(kZonalChunkCells, (long)gm.ds.arr[0] * gm.ds.arr[1] / kZonalChunks);
+    const long cells = std::min<long>(kZonalChunkCells, (long)gm.ds.arr[0] * gm.ds.arr[1] /
+                                                             (ks.form == Form::Focal ? kZonalChunksFocal : kZonalChunksLocal));
     t.L.CH = (int)std::max(1L, cells / (tile.TX * tile.TY));
   }
   return true;
