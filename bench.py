@@ -770,20 +770,10 @@ def main():
         if len(kt) != 1 or launches != args.gens:
             raise SystemExit("bench.py: the profiled step launched %s, expected %d launches of one kernel"
                              % ({k: v["count"] for k, v in kt.items()}, args.gens))
-        # HBM bytes per launch of this kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE
-        # passes scaled by a copy kernel of known size (profiles/life_hbm_traffic.json)
-        traffic = None
-        try:
-            with open(os.path.join(ROOT, "profiles", "life_hbm_traffic.json")) as f:
-                tr = json.load(f)
-            if kname in tr.get("kernels", {}):
-                traffic = tr["kernels"][kname]["bytes_per_launch"]
-        except (OSError, ValueError, KeyError):
-            pass
         alg_bytes = 2.0 * cells  # one U8 read + one U8 write per cell and generation
         achieved = alg_bytes / (kern_ms * 1e-3) / 1e9
         roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                    "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                    "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
                     "kernel": kname, "kernel_avg_ms": round(kern_ms, 5), "kernel_min_ms": round(krec["min_ms"], 5),
                     "launches": launches, "algorithmic_bytes_per_launch": int(alg_bytes)}
     host = M.stats()
