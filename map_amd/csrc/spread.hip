@@ -182,11 +182,21 @@ struct Lds {
   unsigned ticket, tile, served, sum;
 };
 
+// An entry's place is shared: a work-group can wait there with a ticket of a later lap, and an
+// entry put late can meet the next lap's. So it goes into a free place, and out of its place, by
+// compare-and-exchange: no entry is stored over another one or taken twice. Which of the
+// work-groups that wait at a place gets which of its entries does not matter. The place of put n is
+// free in the end: a queue holds a tile once, at most cap in all, so when put n has its number the
+// ticket of put n - cap, and with it a work-group that empties the place, has been taken. (The
+// builtin is the one that both compilers of this text know; its system scope adds nothing to
+// agent scope here, and it is relaxed.)
+__device__ __forceinline__ bool swap_entry(unsigned* slot, unsigned seen, unsigned v) {
+  return __atomic_compare_exchange_n(slot, &seen, v, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+}
 __device__ __forceinline__ void put(const Work& w, unsigned tile) {
   const unsigned q = tile % w.nq;
   unsigned* slot = w.queue + q * w.cap + add_agent(&w.ctl[q * CTL + 1], 1u) % w.cap;
-  while (ld_agent(slot)) nap();  // its taker has the ticket already and is about to free it
-  st_agent(slot, tile + 1u);
+  while (!swap_entry(slot, 0u, tile + 1u)) nap();
 }
 
 // Ring cell k of a tile: -1..TS in x and y.
@@ -490,8 +500,8 @@ __device__ void visits(Lds<T>& L, const T* __restrict__ in, const uint8_t* __res
         unsigned v = first ? k * w.nq + q + 1u : 0u;
         for (int r = 0; !first && v == 0u && r < 16; r++) {
           v = ld_agent(slot);
-          if (v) st_agent(slot, 0u);
-          else nap();
+          if (v && !swap_entry(slot, v, 0u)) v = 0u;
+          if (!v) nap();
         }
         L.tile = v;
         // read before the finished bits: what is notified later is another visit's
