@@ -32,7 +32,8 @@
 // that one lies in a single row or column of blocks: along y its columns are a constant stride
 // apart, and along x, where the rows are a block row apart, a row's K cells move as vectors.
 // (Cell by cell, with a step through the blocks for each, the addresses took more instructions
-// than the columns; that path is left for block sides that K does not divide.)
+// than the columns; that path is left for block sides that K does not divide and for blocks of
+// gigabytes.)
 // 16384^2 F32 from the centre: 2.4 ms, 18.7 us a band (a work-group of 256 rows exchanging
 // columns through LDS with a barrier, cells moved one by one: 4.8 ms; a branch around the
 // operation for inputs that are not finite, and the diagonal's selection in every band:
@@ -344,6 +345,14 @@ static int reach(int s, int ds, int u0, int u1) {  // cells from s to the edge a
   return u > 0 ? ds - 1 - s : s;
 }
 
+// Whether a wavefront's 2 * OWN rows along x lie within 2^32 bytes: LINES keeps their places as 32-bit
+// offsets (a 64-bit address per row, cell and lane would be two more instructions each). They cross
+// into another block column at most once in BS0 cells, a block's cells further on.
+static bool lines_fit(int BS0, int BS1, int NB0, int dt_bytes) {
+  const int rows = 2 * OWN - 1, crossed = (BS0 - 1 + rows) / BS0, most = crossed < NB0 - 1 ? crossed : NB0 - 1;
+  return (uint64_t)((int64_t)most * BS0 * (BS1 - 1) + rows) * (uint64_t)dt_bytes < (1ull << 32);
+}
+
 // dt_bytes 4: float, 8: double; op: 0 sum, 1 prod, 2 max, 3 min. Returns the launch count.
 int run(void* out, const void* in, int dt_bytes, int op, int BS0, int BS1, int NB0, int NB1, int DS0, int DS1, int s0,
         int s1, void* stream) {
@@ -364,7 +373,7 @@ int run(void* out, const void* in, int dt_bytes, int op, int BS0, int BS1, int N
   // bands aligned in x or y lie in one column or row of blocks, and vectors along x are aligned
   for (int o = 0; o < 8; o++) {
     Oct& O = P.oct[o];
-    O.mode = O.fx ? (BS0 % K ? CELLS : O.fx > 0 ? UP : DOWN) : (BS1 % K ? CELLS : LINES);
+    O.mode = O.fx ? (BS0 % K ? CELLS : O.fx > 0 ? UP : DOWN) : (BS1 % K || !lines_fit(BS0, BS1, NB0, dt_bytes) ? CELLS : LINES);
   }
   const bool quick = dt_bytes == 4 && maxL0 <= QUICK_MAX;
   hipStream_t s = (hipStream_t)stream;
