@@ -1138,29 +1138,30 @@ BitRule bit_rule(const Group& g, Node* out) {
   vars.push_back("m.c");
   const std::string e = bool_expr(table, vars, 0);
   std::ostringstream o;
-  o << "#include \"mapx_dev.hiph\"\nnamespace {\nstruct Rule {\n"
+  o << "namespace {\nstruct Rule {\n"
     << "  template <class V> __device__ static __forceinline__ V f(const mx::BitRow<V>& u, const mx::BitRow<V>& m, const mx::BitRow<V>& d) {\n";
   for (size_t i = 0; i < leaves.size(); i++)
     o << "    V p" << i << "[4];\n    mx::win_count<" << leaves[i].rows[0] << ", " << leaves[i].rows[1] << ", "
       << leaves[i].rows[2] << ">(u, m, d, p" << i << ");\n";
   o << "    (void)u; (void)m; (void)d;\n    return " << (e == "0" ? "V(0u)" : e == "1" ? "V(~0u)" : e) << ";\n  }\n};\n}  // namespace\n\n";
-  const std::string K = std::to_string(kBitGens);
+  br.text = o.str();
+  br.name = "bit_" + hex_hash(br.text + dev::header_source());
+  return br;
+}
+
+std::string bit_source(const BitRule& br, int rows) {
+  const std::string K = std::to_string(kBitGens), r = std::to_string(rows);
+  std::ostringstream o;
+  o << "#include \"mapx_dev.hiph\"\n" << br.text;
   auto kernel = [&](const std::string& tail, const std::string& args, const std::string& body) {
-    o << "extern \"C\" __global__ void __launch_bounds__(256) KRN_NAME" << tail << "(" << args << ") {\n  " << body << "\n}\n";
+    o << "extern \"C\" __global__ void __launch_bounds__(256) " << br.name << tail << "(" << args << ") {\n  " << body << "\n}\n";
   };
   kernel("_pack", "const mx::u8* in, mx::u32* out, mx::BitGeo g, mx::u32* bad, mx::u32* not_bits, mx::u32 run",
          "mx::bit_pack(in, out, g, bad, not_bits, run);");
-  for (int rows : kBitRows) {
-    const std::string r = std::to_string(rows);
-    kernel("_step" + r, "const mx::u32* in, mx::u32* out, mx::BitGeo g, int gens, const mx::u32* not_bits, mx::u32 run",
-           "mx::bit_step<Rule, " + r + ", " + K + ">(in, out, g, gens, not_bits, run);");
-  }
+  kernel("_step" + r, "const mx::u32* in, mx::u32* out, mx::BitGeo g, int gens, const mx::u32* not_bits, mx::u32 run",
+         "mx::bit_step<Rule, " + r + ", " + K + ">(in, out, g, gens, not_bits, run);");
   kernel("_unpack", "const mx::u32* in, mx::u8* out, mx::BitGeo g", "mx::bit_unpack(in, out, g);");
-  std::string src = o.str();
-  br.name = "bit_" + hex_hash(src + dev::header_source());
-  for (size_t pos; (pos = src.find("KRN_NAME")) != std::string::npos;) src.replace(pos, 8, br.name);
-  br.source = src;
-  return br;
+  return o.str();
 }
 
 }  // namespace mapx

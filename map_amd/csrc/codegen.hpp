@@ -89,13 +89,16 @@ std::string kernel_shape_key(const Group& g, const std::vector<Node*>& d2_outs, 
 // A focal group that is a 3x3 rule on 0/1 rasters: one U8 raster in, one U8
 // raster out that holds 0 or 1 whenever the input does, through 0/1-weighted
 // window sums, neighbours and integer statements of them and constants.
-// `source` is the module of its bit chain (kernels KRN_pack,
-// KRN_step<rows>, KRN_unpack of device/mapx_dev.hiph's bit chains), "" when the
-// group is none.
+// `text` is the rule as the kernels of device/mapx_dev.hiph's bit chains take it,
+// "" when the group is none.
 struct BitRule {
-  std::string name, source;
+  std::string name, text;
 };
 BitRule bit_rule(const Group& g, Node* out);
+// The module of a bit chain whose wavefronts own `rows` rows: kernels <name>_pack,
+// <name>_step<rows>, <name>_unpack. (One module per shape: with hipcc on
+// this machine's CPU 4 rows take 2.4 s, 16 rows 3.5, 80 rows 9.3.)
+std::string bit_source(const BitRule& r, int rows);
 constexpr int kBitGens = 8;                      // generations of one step launch
 constexpr int kBitRows[] = {4, 16, 80};          // rows a wavefront of a step kernel owns
 constexpr int kBitShapes = sizeof(kBitRows) / sizeof(kBitRows[0]);

@@ -1608,28 +1608,49 @@ void Runtime::find_bit_chains(Plan& plan) {
     }
     if (c.groups.size() < kBitChain) continue;
     for (const Group* h : c.groups) taken.insert(h);
-    auto known = bit_kernels_.find(key);
-    if (known == bit_kernels_.end()) {
-      if (bit_kernels_.size() >= 4096) bit_kernels_.clear();  // bounded; plans keep theirs
-      HostTimer ht(cnt.ms_codegen);
-      auto k = std::make_shared<BitKernels>();
-      const BitRule br = bit_rule(*c.groups[0], c.out[0]);
-      if (!br.source.empty()) {
-        k->name = br.name;
-        k->pack = dev::function(br.source, br.name + "_pack").fn;
-        for (int i = 0; i < kBitShapes; i++)
-          k->step[i] = dev::function(br.source, br.name + "_step" + std::to_string(kBitRows[i])).fn;
-        k->unpack = dev::function(br.source, br.name + "_unpack").fn;
-        kernel_src_[br.name] = br.source;
-        cnt.compiles++;
-      }
-      known = bit_kernels_.emplace(key, std::move(k)).first;
-    }
-    if (!known->second->unpack) continue;  // no bit rule
-    c.k = known->second;
+    if (bit_kernels_.size() >= 4096) bit_kernels_.clear();  // bounded; plans keep theirs
+    auto& k = bit_kernels_[key];
+    if (!k) k = std::make_shared<BitKernels>();
+    c.k = k;
     for (size_t i = 0; i < c.groups.size(); i++) plan.chain_at[c.groups[i]] = {plan.chains.size(), i};
     plan.chains.push_back(std::move(c));
   }
+}
+
+namespace {
+// Rows a wavefront owns: it computes 2 * kBitGens more, and the SIMD with the
+// most wavefronts decides the time of a launch. Index into kBitRows, and the wavefronts.
+std::pair<int, long> bit_shape(const Meta& m) {
+  const long nsx = ((m.ds.arr[0] + 31L) / 32 + 61) / 62, simds = 4L * std::max(1, dev::num_cus());
+  int shape = 0;
+  long waves = 0, best = 0;
+  for (int i = 0; i < kBitShapes; i++) {
+    const long w = nsx * ((m.ds.arr[1] + kBitRows[i] - 1L) / kBitRows[i]);
+    const long cost = ((w + simds - 1) / simds) * (kBitRows[i] + 2 * kBitGens);
+    if (i == 0 || cost < best) { best = cost; waves = w; shape = i; }
+  }
+  return {shape, waves};
+}
+}  // namespace
+
+// The kernels of a chain for one shape, null when its groups are no bit rule.
+// Looked up and compiled when a chain is about to run, so that a script whose
+// chains never pay, or run another way, waits for neither.
+const Runtime::BitKernels::Shape* Runtime::bit_kernels(const BitChain& c, int shape) {
+  BitKernels& k = *c.k;
+  BitKernels::Shape& s = k.shape[shape];
+  if (s.unpack) return &s;
+  HostTimer ht(cnt.ms_codegen);
+  if (!k.asked) k.rule = bit_rule(*c.groups[0], c.out[0]);
+  k.asked = true;
+  if (k.rule.text.empty()) return nullptr;
+  const std::string src = bit_source(k.rule, kBitRows[shape]);
+  s.pack = dev::function(src, k.rule.name + "_pack").fn;
+  s.step = dev::function(src, k.rule.name + "_step" + std::to_string(kBitRows[shape])).fn;
+  s.unpack = dev::function(src, k.rule.name + "_unpack").fn;
+  kernel_src_[k.rule.name] = src;
+  cnt.compiles++;
+  return &s;
 }
 
 // Groups first..first+n-1 of a chain: the last one's raster from the first
@@ -1641,6 +1662,8 @@ void Runtime::launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t
   Node* on = c.out[first + n - 1];
   ensure_input(in);
   const Meta& m = on->meta;
+  const auto [shape, waves] = bit_shape(m);
+  const BitKernels::Shape& k = c.k->shape[shape];
   void* out = store.alloc(rasterBytes(m));
   resident_[on] = out;
   BitGeoHost g{m.ds.arr[0], m.ds.arr[1], (m.ds.arr[0] + 31) / 32, m.bs.arr[0], m.bs.arr[1], m.nb(0)};
@@ -1660,7 +1683,7 @@ void Runtime::launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t
     for (auto& x : args) { p.push_back(x.first); z.push_back(x.second); }
     dev::Function f;
     f.fn = fn;
-    f.name = c.k->name + tail;
+    f.name = c.k->rule.name + tail;
     dev::launch(f, grid, 256, p.data(), z.data(), (int)p.size());
     cnt.launches++;
   };
@@ -1668,25 +1691,15 @@ void Runtime::launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t
   const unsigned pgrid = (unsigned)((spots + 255) / 256);
   void *bad = bit_flags_ + slot, *not_bits = bit_runs_ + slot;
   uint32_t run = ++bit_run_;
-  launch(c.k->pack, "_pack", pgrid, {{&src, 8}, {&a, 8}, {&g, sizeof g}, {&bad, 8}, {&not_bits, 8}, {&run, 4}});
-  // Rows a wavefront owns: it computes 2 * kBitGens more, and the SIMD with the
-  // most wavefronts decides the time of a launch.
-  const long nsx = (g.WD + 61) / 62, simds = 4L * std::max(1, dev::num_cus());
-  int shape = 0;
-  long waves = 0, best = 0;
-  for (int i = 0; i < kBitShapes; i++) {
-    const long w = nsx * ((g.H + kBitRows[i] - 1L) / kBitRows[i]);
-    const long cost = ((w + simds - 1) / simds) * (kBitRows[i] + 2 * kBitGens);
-    if (i == 0 || cost < best) { best = cost; waves = w; shape = i; }
-  }
+  launch(k.pack, "_pack", pgrid, {{&src, 8}, {&a, 8}, {&g, sizeof g}, {&bad, 8}, {&not_bits, 8}, {&run, 4}});
   const std::string step = "_step" + std::to_string(kBitRows[shape]);
   for (size_t done = 0; done < n; done += kBitGens) {
     int gens = (int)std::min<size_t>(kBitGens, n - done);
-    launch(c.k->step[shape], step.c_str(), (unsigned)((waves + 3) / 4), 
+    launch(k.step, step.c_str(), (unsigned)((waves + 3) / 4),
            {{&a, 8}, {&b, 8}, {&g, sizeof g}, {&gens, 4}, {&not_bits, 8}, {&run, 4}});
     std::swap(a, b);
   }
-  launch(c.k->unpack, "_unpack", pgrid, {{&a, 8}, {&out, 8}, {&g, sizeof g}});
+  launch(k.unpack, "_unpack", pgrid, {{&a, 8}, {&out, 8}, {&g, sizeof g}});
 }
 
 // Measured, one evaluation of n generations, chain against groups: 256^2 cells
@@ -1709,6 +1722,7 @@ void Runtime::run_bit_chains(Eval& e, size_t level) {
     auto it = e.plan->chain_at.find(g);
     if (it == e.plan->chain_at.end() || e.not_bits.count(g)) continue;
     const BitChain& c = e.plan->chains[it->second.first];
+    if (c.k->asked && c.k->rule.text.empty()) continue;  // no bit rule
     // from here as far as nobody keeps or asks for a raster between
     size_t i = it->second.second, n = 0;
     while (i + n < c.groups.size()) {
@@ -1720,7 +1734,8 @@ void Runtime::run_bit_chains(Eval& e, size_t level) {
       n++;
       if (ext_refs(outs[0]) > 0 || e.tset.count(outs[0])) break;
     }
-    if (n >= kBitChain && bit_chain_pays(n, c.out[i]->meta)) runs.push_back({&c, i, n});
+    if (n >= kBitChain && bit_chain_pays(n, c.out[i]->meta) && bit_kernels(c, bit_shape(c.out[i]->meta).first))
+      runs.push_back({&c, i, n});
   }
   if (runs.empty()) return;
   PauseRecording pause;
@@ -2077,7 +2092,7 @@ std::string Runtime::plan(const std::vector<Node*>& targets_in) {
     }
     if (pattern_is(g->pat, FOCAL) && chain_input(*g) && chain_output(*g)) {
       const BitRule br = bit_rule(*g, chain_output(*g));
-      if (!br.source.empty()) j << ", \"bit_rule\": \"" << esc(br.source) << "\"";
+      if (!br.text.empty()) j << ", \"bit_rule\": \"" << esc(bit_source(br, kBitRows[kBitShapes - 1])) << "\"";
     }
     if (!host_group(*g)) {
       std::vector<Node*> outs = d2_outputs(*g, tsorted), kouts;

@@ -224,16 +224,18 @@ class Runtime {
   // A sequence of groups that apply one bit rule (codegen's bit_rule), each to
   // the raster of the one before and to nothing else.
   struct BitKernels {
-    std::string name;
-    void *pack = nullptr, *step[kBitShapes] = {}, *unpack = nullptr;
+    bool asked = false;  // whether the groups are a bit rule is known
+    BitRule rule;        // without text when they are none
+    struct Shape { void *pack = nullptr, *step = nullptr, *unpack = nullptr; } shape[kBitShapes];  // as compiled
   };
   struct BitChain {
     std::vector<const Group*> groups;
     std::vector<Node*> out;  // the raster of each group
     Node* in = nullptr;      // the first group's input
-    std::shared_ptr<const BitKernels> k;
+    std::shared_ptr<BitKernels> k;
   };
-  std::unordered_map<std::string, std::shared_ptr<BitKernels>> bit_kernels_;  // by rule; no kernels: no bit rule
+  std::unordered_map<std::string, std::shared_ptr<BitKernels>> bit_kernels_;  // by rule
+  const BitKernels::Shape* bit_kernels(const BitChain& c, int shape);
   void find_bit_chains(Plan& plan);
   void run_bit_chains(Eval& e, size_t level);
   void launch_bit_chain(const BitChain& c, size_t first, size_t n, size_t slot);

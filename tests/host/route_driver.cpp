@@ -1,0 +1,161 @@
+// Which kernels the runtime compiles and launches, and what memory it takes for them, on the
+// device double (dev_double.cpp, compiled into this file behind hooks on its compilation, launch
+// and allocation entries) through the C ABI. One scenario per run: route_driver NAME.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "dev.hpp"
+
+#define function function_double
+#define launch launch_double
+#include "dev_double.cpp"
+#undef function
+#undef launch
+
+#include "../../include/mapx.h"
+
+namespace {
+struct Launched {
+  std::string name;
+  unsigned grid, grid_y;
+};
+std::vector<std::string> compiled;  // kernels asked for, in order
+std::map<std::string, std::string> sources;
+std::vector<Launched> launched;
+std::function<void(const Launched&, void**, const size_t*, int)> on_launch;
+}  // namespace
+
+namespace mapx {
+namespace dev {
+Function function(const std::string& source, const std::string& name) {
+  compiled.push_back(name);
+  sources[name] = source;
+  return function_double(source, name);
+}
+void launch(const Function& f, unsigned grid, unsigned block, void** params, const size_t* sizes, int n, unsigned grid_y) {
+  launched.push_back({f.name, grid, grid_y});
+  if (on_launch) on_launch(launched.back(), params, sizes, n);
+  launch_double(f, grid, block, params, sizes, n, grid_y);
+}
+}  // namespace dev
+}  // namespace mapx
+
+namespace {
+
+enum { F32 = 1, U8 = 4, S32 = 10, ROWBLK = 3, DEV_GPU = 4, GT = 9 };
+
+[[noreturn]] void fail(const std::string& what) {
+  std::fprintf(stderr, "route driver: %s (%s)\n", what.c_str(), ma_lastError());
+  std::exit(2);
+}
+void expect(bool ok, const std::string& what) {
+  if (!ok) fail(what);
+}
+bool ends(const std::string& s, const std::string& tail) {
+  return s.size() >= tail.size() && s.compare(s.size() - tail.size(), tail.size(), tail) == 0;
+}
+bool has(const std::string& s, const std::string& part) { return s.find(part) != std::string::npos; }
+int kernels(const std::vector<std::string>& v, const std::string& part) {
+  int n = 0;
+  for (auto& s : v) n += has(s, part);
+  return n;
+}
+int launches(const std::string& part) {
+  int n = 0;
+  for (auto& l : launched) n += has(l.name, part);
+  return n;
+}
+
+// A held node, as a program holds one.
+struct R {
+  ma_node_t* n = nullptr;
+  R() {}
+  explicit R(ma_node_t* p) : n(p) {
+    expect(n != nullptr, "factory");
+    ma_increaseRef(n);
+  }
+  R(const R& o) : n(o.n) { if (n) ma_increaseRef(n); }
+  R& operator=(const R& o) {
+    if (o.n) ma_increaseRef(o.n);
+    if (n) ma_decreaseRef(n);
+    n = o.n;
+    return *this;
+  }
+  ~R() { if (n) ma_decreaseRef(n); }
+};
+ma_dim2_t dim(int a, int b) { ma_dim2_t d; d.arr[0] = a; d.arr[1] = b; d.n = 2; return d; }
+ma_dim2_t none() { ma_dim2_t d; d.arr[0] = 0; d.arr[1] = 0; d.n = 0; return d; }
+ma_variant_t s32(int v) { ma_variant_t x; std::memset(&x, 0, sizeof x); x.u.s32 = v; x.dtype = S32; return x; }
+R input(int w, int h, int bs, int dt, int size) {
+  const size_t n = (size_t)((w + bs - 1) / bs) * ((h + bs - 1) / bs) * bs * bs * size;
+  std::vector<char> a(n, 0);
+  return R(ma_input(a.data(), n, dim(w, h), dt, dim(bs, bs)));
+}
+R conv(const R& a, const std::vector<int>& w) {
+  std::vector<ma_variant_t> v;
+  for (int x : w) v.push_back(s32(x));
+  return R(ma_convolution(a.n, v.data(), (int)v.size(), dim(3, 3)));
+}
+// n generations of a 0/1 rule: more than `over` of the nine cells
+R rule(R s, int n, int over = 4, int weight = 1) {
+  for (int g = 0; g < n; g++) {
+    R k(ma_constant(s32(over), none(), S32, ROWBLK, none()));
+    R many(ma_binary(conv(s, std::vector<int>(9, weight)).n, k.n, GT));
+    s = R(ma_cast(many.n, U8));
+  }
+  return s;
+}
+void eval(const std::vector<R>& v) {
+  std::vector<ma_node_t*> p;
+  for (const R& r : v) p.push_back(r.n);
+  ma_eval(p.data(), (int)p.size());
+  if (std::strlen(ma_lastError())) fail("eval");
+}
+
+// The module of a chain of 0/1 rules is compiled when a chain runs, for the shape it runs with.
+void scenario_compile() {
+  eval({rule(input(300, 200, 64, U8, 1), 3)});  // too short to pay
+  expect(kernels(compiled, "bit_") == 0, "kernels compiled for a chain that does not pay");
+  expect(launches("_pack") == 0, "a chain that does not pay ran");
+  ma_setOption("form", 0);
+  eval({rule(input(300, 200, 64, U8, 1), 40)});
+  ma_setOption("form", 1);
+  ma_setOption("tile_tx", 256); ma_setOption("tile_ty", 16); ma_setOption("tile_vx", 4);
+  eval({rule(input(300, 200, 64, U8, 1), 40)});
+  ma_setOption("tile_tx", 0); ma_setOption("tile_ty", 0); ma_setOption("tile_vx", 0);
+  expect(kernels(compiled, "bit_") == 0, "kernels compiled for chains that run by groups");
+  eval({rule(input(300, 200, 64, U8, 1), 40, 4, 2)});
+  expect(kernels(compiled, "bit_") == 0, "kernels compiled for groups that are no bit rule");
+  eval({rule(input(300, 200, 64, U8, 1), 40)});
+  expect(launches("_pack") == 1 && launches("_step") == 5 && launches("_unpack") == 1, "a chain of 40 generations");
+  expect(kernels(compiled, "_step") == 1, "more than one shape compiled");
+  const size_t n = compiled.size();
+  eval({rule(input(310, 190, 64, U8, 1), 40)});  // the same rule and shape on another raster
+  expect(compiled.size() == n && launches("_pack") == 2, "compiled again for another raster");
+  eval({rule(input(4000, 4000, 512, U8, 1), 24)});
+  expect(kernels(compiled, "_step") == 2 && launches("_pack") == 3, "the shape of a large raster");
+  for (auto& s : sources)
+    if (has(s.first, "_step")) {
+      size_t steps = 0;
+      for (size_t p = 0; (p = s.second.find("mx::bit_step<", p)) != std::string::npos; p++) steps++;
+      expect(steps == 1, "a module holds more than one step kernel");
+    }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}};
+  if (argc != 2 || !all.count(argv[1])) return 3;
+  ma_setupDevices("", DEV_GPU, "");
+  all.at(argv[1])();
+  std::printf("route driver: ok\n");
+  return 0;
+}
