@@ -1578,7 +1578,11 @@ long bit_spots(const Meta& m) { return 2L * ((m.ds.arr[0] + 31) / 32) * ((m.ds.a
 constexpr size_t kBitFlags = 1024;                   // chains of one level that run together
 }  // namespace
 
+// Looked for when a plan is first evaluated, not when it is made: a request of
+// the server runs by groups, and its plan may be evaluated later.
 void Runtime::find_bit_chains(Plan& plan) {
+  HostTimer ht(cnt.ms_plan);
+  plan.chained = true;
   std::unordered_map<Node*, std::vector<const Group*>> readers;
   for (auto& g : plan.groups)
     for (Node* n : g->ins)
@@ -1898,7 +1902,6 @@ void Runtime::eval_plan(Eval& e) {
       HostTimer ht(cnt.ms_fuse);
       pl->groups = Fuser(fo).fuse(e.list);
     }
-    if (!serving()) find_bit_chains(*pl);
     pit = plans_.emplace(pkey, std::move(pl)).first;
   }
   e.plan = pit->second;
@@ -1985,6 +1988,7 @@ void Runtime::evaluate(const std::vector<Node*>& targets) {
     ~Uncut() { r->eval_uncut(e); }
   } uncut{this, e};
   eval_plan(e);
+  if (!e.plan->chained) find_bit_chains(*e.plan);
   // the evaluation's rasters stay in HBM while it runs (spill_one passes them over)
   struct Live {
     Runtime* r; unsigned long long t;

@@ -245,6 +245,7 @@ class Runtime {
   uint32_t bit_run_ = 0;           // number of the last run
   struct Plan {
     std::vector<std::unique_ptr<Group>> groups;
+    bool chained = false;  // the chains have been looked for
     std::vector<BitChain> chains;
     std::unordered_map<const Group*, std::pair<size_t, size_t>> chain_at;  // group -> (chain, place in it)
     std::map<std::pair<const Group*, std::vector<Node*>>, KernelEntry> kernels;

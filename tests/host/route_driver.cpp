@@ -149,10 +149,35 @@ void scenario_compile() {
     }
 }
 
+void serve(const std::vector<R>& v) {
+  std::vector<ma_node_t*> p;
+  for (const R& r : v) p.push_back(r.n);
+  if (ma_serveSubmit(p.data(), (int)p.size()) < 0) fail("serveSubmit");
+  for (int i = 0; i < 1000; i++) {
+    if (ma_serveStep(0) < 0) fail("serveStep");
+    long long id;
+    double a, b, c;
+    if (ma_serveTake(&id, &a, &b, &c, 1) == 1) return;
+  }
+  fail("a request that does not complete");
+}
+
+// A plan made for a request of the server has its chains when it is evaluated later.
+void scenario_served_plan() {
+  R s = rule(input(300, 200, 64, U8, 1), 40);
+  if (ma_serveOpen(64LL << 20, 8) != 0) fail("serveOpen");
+  serve({s});
+  if (ma_serveClose() != 0) fail("serveClose");
+  expect(launches("_pack") == 0, "the served form runs by groups");
+  ma_release(s.n);
+  eval({s});
+  expect(launches("_pack") == 1 && launches("_step") == 5, "the plan of a served request has no chain");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}};
+  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}};
   if (argc != 2 || !all.count(argv[1])) return 3;
   ma_setupDevices("", DEV_GPU, "");
   all.at(argv[1])();
