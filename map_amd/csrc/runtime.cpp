@@ -1502,8 +1502,10 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
 // (device/mapx_dev.hiph, bit chains) and only the last raster is written.
 // The input may hold values above 1, for which the bits are not the raster:
 // the pack kernel reports them (the steps then end at once), the host waits for
-// the sequence and, where a value was reported, runs the groups one by one as
-// if there were no chain.
+// the sequence and, where a value was reported, runs its first group as if there
+// were no chain. What that group computes is a 0/1 raster for most rules, so the
+// sequence is tried once more from there; and the plan keeps the place, so that
+// its next evaluation does not look at the same raster again.
 
 namespace {
 // One 0/1 raster in and out, and nothing else of a D2 shape: the cheap part of
@@ -1720,12 +1722,13 @@ bool Runtime::bit_chain_pays(size_t n, const Meta& m) {
 // later ones) and marks the groups they computed in `e.done`.
 void Runtime::run_bit_chains(Eval& e, size_t level) {
   if (opt.form == FORM_PLAIN || opt.tile.TX > 0 || e.plan->chains.empty()) return;
-  struct Run { const BitChain* c; size_t first, n; };
+  struct Run { BitChain* c; size_t first, n; };
   std::vector<Run> runs;
   for (const Group* g : e.levels[level]) {
     auto it = e.plan->chain_at.find(g);
-    if (it == e.plan->chain_at.end() || e.not_bits.count(g)) continue;
-    const BitChain& c = e.plan->chains[it->second.first];
+    if (it == e.plan->chain_at.end()) continue;
+    BitChain& c = e.plan->chains[it->second.first];
+    if (it->second.second < c.from) continue;
     if (c.k->asked && c.k->rule.text.empty()) continue;  // no bit rule
     // from here as far as nobody keeps or asks for a raster between
     size_t i = it->second.second, n = 0;
@@ -1765,7 +1768,7 @@ void Runtime::run_bit_chains(Eval& e, size_t level) {
         Node* on = x.c->out[x.first + x.n - 1];
         store.release(resident_.at(on));
         resident_.erase(on);
-        for (size_t i = 0; i < x.n; i++) e.not_bits.insert(x.c->groups[x.first + i]);
+        x.c->from = x.c->from ? x.c->groups.size() : x.first + 1;
       } else {
         cnt.groups += (long)x.n;
         for (size_t i = 0; i < x.n; i++) e.done.insert(x.c->groups[x.first + i]);

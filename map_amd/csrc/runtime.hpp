@@ -174,7 +174,6 @@ class Runtime {
     std::unordered_map<Node*, int> uses;
     std::unordered_set<Node*> tset;
     std::unordered_set<const Group*> done;      // groups a bit chain has computed
-    std::unordered_set<const Group*> not_bits;  // groups of a chain whose input was not 0/1
     // kernels fixed at planning time (requests of the server run later)
     std::unordered_map<const Group*, std::pair<std::vector<Node*>, KernelEntry*>> kern;
   };
@@ -232,6 +231,7 @@ class Runtime {
     std::vector<const Group*> groups;
     std::vector<Node*> out;  // the raster of each group
     Node* in = nullptr;      // the first group's input
+    size_t from = 0;         // the groups before this one read no 0/1 raster when the chain was tried
     std::shared_ptr<BitKernels> k;
   };
   std::unordered_map<std::string, std::shared_ptr<BitKernels>> bit_kernels_;  // by rule

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -174,10 +175,41 @@ void scenario_served_plan() {
   expect(launches("_pack") == 1 && launches("_step") == 5, "the plan of a served request has no chain");
 }
 
+// Rasters that hold more than 0 and 1: the pack kernels of `bad` say so.
+void report(const std::vector<bool>& bad) {
+  auto n = std::make_shared<size_t>(0);
+  launched.clear();
+  on_launch = [=](const Launched& l, void** params, const size_t*, int) {
+    if (!ends(l.name, "_pack")) return;
+    if (*n < bad.size() && bad[*n]) **(unsigned**)params[3] = 1;  // its word in pinned memory
+    ++*n;
+  };
+}
+void scenario_no_bits() {
+  R in = input(300, 200, 64, U8, 1), s = rule(in, 40);
+  auto groups = [] { return (int)launched.size() - launches("bit_"); };
+  report({true});
+  eval({s});
+  expect(launches("_pack") == 2 && groups() == 1, "the generations after the first one are a chain");
+  ma_release(s.n);
+  report({});
+  eval({s});
+  expect(launches("_pack") == 1 && groups() == 1, "the second evaluation looks at the same raster again");
+  R t = rule(in, 41, 3);
+  report({true, true, true});
+  eval({t});
+  expect(launches("_pack") == 2 && groups() == 41, "rasters that are never 0/1 run by groups");
+  ma_release(t.n);
+  report({});
+  eval({t});
+  expect(launches("_pack") == 0 && groups() == 41, "rasters that are never 0/1 are tried again");
+  on_launch = nullptr;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}};
+  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}, {"no bits", scenario_no_bits}};
   if (argc != 2 || !all.count(argv[1])) return 3;
   ma_setupDevices("", DEV_GPU, "");
   all.at(argv[1])();
