@@ -1,6 +1,7 @@
 #include "runtime.hpp"
 #include "rasterio.hpp"
 #include "dev.hpp"
+#include "spread.hpp"
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -20,10 +21,6 @@ int run(void* out, const void* in, int dt_bytes, int op, int BS0, int BS1, int N
 namespace gen {  // gen.hip
 void nalloc_scratch_init(int device);
 }  // namespace gen
-namespace spread {  // spread.hip
-int run(void* out, const void* in, const void* dir, void* cnt, int dt, int BS0, int BS1, int NB0, int NB1, int DS0,
-        int DS1, void* stream);
-}  // namespace spread
 }  // namespace mapx
 
 namespace mapx {
@@ -1171,9 +1168,7 @@ void Runtime::spread_task(const Group& g, Eval& e) {
   const Meta& m = n->meta;
   void* out = store.alloc(rasterBytes(m));
   resident_[n] = out;
-  // per 64x64 tile: 17 bits per cell, a notification word and a queue entry; the queues' counters
-  const size_t tiles = (size_t)((m.ds.arr[0] + 63) / 64) * ((m.ds.arr[1] + 63) / 64);
-  void* scratch = store.alloc(tiles * (8192 + 512 + 8) + 64 * 256 + 64 * 4);
+  void* scratch = store.alloc(spread::scratch_bytes(m.ds.arr[0], m.ds.arr[1]));
   PauseRecording pause;
   cnt.launches += spread::run(out, residentPtr(n->prev[0]), residentPtr(n->prev[1]), scratch, m.dt, m.bs.arr[0],
                               m.bs.arr[1], m.nb(0), m.nb(1), m.ds.arr[0], m.ds.arr[1], dev::stream());

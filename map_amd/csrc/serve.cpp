@@ -14,6 +14,7 @@
 // request is still computing waits for that request.
 #include "dev.hpp"
 #include "runtime.hpp"
+#include "spread.hpp"
 #include <chrono>
 #include <deque>
 #include <sstream>
@@ -189,11 +190,11 @@ int Runtime::serveStep(int wait_us) {
         if (host_group(*g)) continue;
         Node* rn = radial_node(*g);
         Node* sn = spread_node(*g);
-        if (rn || sn) {  // no generated kernel: its output raster (and a spread's count words)
+        if (rn || sn) {  // no generated kernel: its output raster (and a spread's scratch)
           bool z = false;
           const Meta& m = (rn ? rn : sn)->meta;
           if (!kernel_outputs(*g, e.tsorted, z).empty())
-            fp += rasterBytes(m) + (sn ? (size_t)m.bs.arr[0] * m.bs.arr[1] * m.nb(0) * m.nb(1) * 8 + 8 : 0);
+            fp += rasterBytes(m) + (sn ? spread::scratch_bytes(m.ds.arr[0], m.ds.arr[1]) : 0);
           for (Node* n : g->ins) {
             if (n->meta.nd == D2 && spilled_.count(n)) unspill(n);
             if (n->meta.nd == D2 && resident_.count(n)) pins.push_back(n);

@@ -40,6 +40,8 @@
 // stands for a cell that has just finished, so the visits end. Cells on a
 // direction cycle never have all their upstream totals; the last kernel gives
 // them the 0 (the reference's iteration does not end for them).
+#include "spread.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -571,6 +573,8 @@ static void launch(void* out, const void* in, const void* dir, void* scratch, co
   w.ctl = w.done + (size_t)tiles * (TS * 2);
   w.pend = w.ctl + MAX_QUEUES * CTL;
   w.queue = w.pend + tiles;
+  if ((size_t)((char*)(w.queue + (size_t)w.nq * w.cap) - (char*)scratch) > scratch_bytes(g.DS0, g.DS1))
+    throw std::runtime_error("spread: the scratch is too small");
   // (at least nq * cap <= tiles + nq entries and nq * CTL counters to clear)
   const unsigned grid = (unsigned)(((size_t)tiles * (TS * 2) + MAX_QUEUES * CTL + NT - 1) / NT);
   hipLaunchKernelGGL(k_start, dim3(grid), dim3(NT), 0, s, w);
@@ -581,9 +585,6 @@ static void launch(void* out, const void* in, const void* dir, void* scratch, co
   check(hipGetLastError(), "spread cycle launch");
 }
 
-// dt: the DataTypeEnum of the raster.
-// scratch: per 64x64 tile of the raster 8192 bytes of cell words, 512 of finished bits, a notification word and
-// a queue entry (4 bytes each); 64 * 256 bytes of counters and 64 * 4 of queue entries. Returns the launch count.
 int run(void* out, const void* in, const void* dir, void* scratch, int dt, int BS0, int BS1, int NB0, int NB1, int DS0,
         int DS1, void* stream) {
   if (BS0 <= 0 || BS1 <= 0 || NB0 <= 0 || NB1 <= 0 || DS0 <= 0 || DS1 <= 0 || DS0 > NB0 * BS0 || DS1 > NB1 * BS1)

@@ -16,7 +16,9 @@
 
 #define function function_double
 #define launch launch_double
+#define spread spread_double
 #include "dev_double.cpp"
+#undef spread
 #undef function
 #undef launch
 
@@ -46,11 +48,20 @@ void launch(const Function& f, unsigned grid, unsigned block, void** params, con
   launch_double(f, grid, block, params, sizes, n, grid_y);
 }
 }  // namespace dev
+namespace spread {
+// cell words and finished bits, a notification word and a queue entry per 64x64 tile; counters
+size_t needs(int w, int h) { return (size_t)((w + 63) / 64) * ((h + 63) / 64) * (8192 + 512 + 8) + 64 * 256 + 64 * 4; }
+int run(void*, const void*, const void*, void* scratch, int, int, int, int, int, int DS0, int DS1, void*) {
+  const std::vector<char> z(needs(DS0, DS1));
+  dev::h2d(scratch, z.data(), z.size());
+  return 3;
+}
+}  // namespace spread
 }  // namespace mapx
 
 namespace {
 
-enum { F32 = 1, U8 = 4, S32 = 10, ROWBLK = 3, DEV_GPU = 4, GT = 9 };
+enum { F32 = 1, U8 = 4, S32 = 10, ROWBLK = 3, DEV_GPU = 4, SUM = 1, GT = 9 };
 
 [[noreturn]] void fail(const std::string& what) {
   std::fprintf(stderr, "route driver: %s (%s)\n", what.c_str(), ma_lastError());
@@ -175,6 +186,24 @@ void scenario_served_plan() {
   expect(launches("_pack") == 1 && launches("_step") == 5, "the plan of a served request has no chain");
 }
 
+// A served flow accumulation is admitted with the memory it takes: its raster and the scan's scratch.
+void scenario_served_flow() {
+  for (auto& c : std::vector<std::pair<int, int>>{{40, 30}, {700, 500}}) {
+    const int w = c.first, h = c.second, bs = 32;
+    R rain = input(w, h, bs, F32, 4), dir = input(w, h, bs, U8, 1);
+    eval({rain, dir});
+    if (ma_serveOpen(64LL << 20, 8) != 0) fail("serveOpen");
+    R acc(ma_spreadScan(rain.n, dir.n, SUM));
+    serve({acc});
+    const char* p = std::strstr(ma_serveStats(), "\"peak_inflight_bytes\": ");
+    expect(p != nullptr, "serveStats");
+    const size_t got = std::strtoull(p + 23, nullptr, 10);
+    const size_t need = (size_t)((w + bs - 1) / bs) * ((h + bs - 1) / bs) * bs * bs * 4 + mapx::spread::needs(w, h);
+    expect(got == need, "admitted with " + std::to_string(got) + " bytes, takes " + std::to_string(need));
+    if (ma_serveClose() != 0) fail("serveClose");
+  }
+}
+
 // Rasters that hold more than 0 and 1: the pack kernels of `bad` say so.
 void report(const std::vector<bool>& bad) {
   auto n = std::make_shared<size_t>(0);
@@ -209,7 +238,8 @@ void scenario_no_bits() {
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}, {"no bits", scenario_no_bits}};
+  const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}, {"no bits", scenario_no_bits},
+                                                      {"served flow", scenario_served_flow}};
   if (argc != 2 || !all.count(argv[1])) return 3;
   ma_setupDevices("", DEV_GPU, "");
   all.at(argv[1])();
