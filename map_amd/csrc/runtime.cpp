@@ -846,7 +846,16 @@ uint32_t morton2(uint32_t x, uint32_t y) {
 // and 264. Cell-wise groups wait for HBM, and long runs read it better: an overlay
 // of 8191x6001 took 175 us in a 512th and 186 in a 2048th, of 3000x2500 75 in
 // chunks of 65536 cells and 30 in a 512th.
-constexpr int kZonalChunkCells = 65536, kZonalChunksFocal = 2048, kZonalChunksLocal = 512;
+// With many zones the records (24 bytes a zone) outweigh the cells: above 4 bytes
+// of record a cell the raster has one chunk per CU. Slope with statistics of 3000
+// zones, kernel + fold, in a 2048th of the raster / in a 256th / in chunks of 65536
+// cells: 4096^2 233 + 34 / 156 + 7 / 156 + 7 us, 2048^2 107 + 23 / 92 + 8 / 275 + 6,
+// 16 of 2048^2 in a batch 1414 + 246 / 1064 + 89 / 1094 + 16. (64 of 1024^2 in a batch
+// 2860 + 220 / the same / 2250 + 20, where a raster alone takes 60 + 7 and 540 + 6.)
+constexpr int kZonalChunkCells = 65536, kZonalChunksFocal = 2048, kZonalChunksLocal = 512, kZonalChunksMany = 256;
+constexpr long kZonalRecordPerCell = 4;
+// Records of one batched launch: more tasks go in several launches.
+constexpr size_t kZonalRecordBytes = (size_t)512 << 20;
 // Tiles per chunk of other groups: consecutive tiles of a block run on one
 // work-group (halo rows shared with the previous tile are still in L2), at
 // most kChunkTiles. Batches, whose tasks differ, take chunks from the queue: at
@@ -1232,9 +1241,10 @@ bool Runtime::prepare_task(const Group& g, Eval& e, Task& t) {
   const int BS0 = gm.bs.arr[0], BS1 = gm.bs.arr[1], NB0 = gm.nb(0), NB1 = gm.nb(1);
   t.L = HostLaunch{BS0, BS1, NB0, NB1, gm.ds.arr[0], gm.ds.arr[1], -1, 1, 1, 1, 1, 1, 0};
   if (!ks.zouts.empty()) {
-    const long cells = std::min<long>(kZonalChunkCells, (long)gm.ds.arr[0] * gm.ds.arr[1] /
-                                                             (ks.form == Form::Focal ? kZonalChunksFocal : kZonalChunksLocal));
-    t.L.CH = (int)std::max(1L, cells / (tile.TX * tile.TY));
+    const long tc = (long)tile.TX * tile.TY, all = (long)gm.ds.arr[0] * gm.ds.arr[1];
+    auto tiles = [&](long chunks) { return std::max(1L, std::min<long>(kZonalChunkCells, all / chunks) / tc); };
+    t.L.CH = (int)tiles(ks.form == Form::Focal ? kZonalChunksFocal : kZonalChunksLocal);
+    if ((long)ks.part_bytes > kZonalRecordPerCell * t.L.CH * tc) t.L.CH = std::max(t.L.CH, (int)tiles(kZonalChunksMany));
   }
   return true;
 }
@@ -1378,9 +1388,55 @@ void Runtime::fold_results(const std::vector<Task*>& batch, void* parts, void* t
   store.release(res);
 }
 
+// The partial records of one task. Where the store cannot give them, the task
+// takes chunks of 65536 cells: fewer records, and sums that round in another order.
+void* Runtime::zonal_records(Task& t) {
+  const KernelSpec& ks = t.ke->spec;
+  try {
+    return store.alloc((size_t)t.nchunks * ks.part_bytes);
+  } catch (const std::exception&) {
+    const int ch = std::max(1, kZonalChunkCells / (ks.tile.TX * ks.tile.TY));
+    if (t.L.CH >= ch) throw;
+    t.L.CH = ch;
+    t.chunking(0);
+    return store.alloc((size_t)t.nchunks * ks.part_bytes);
+  }
+}
+
 // Launches a batch of tasks of one kernel: per block (plain form), one task by
 // value, or many tasks from a device task table with a device chunk queue.
 void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* async) {
+  if (batch.size() > 1 && opt.form != FORM_PLAIN && !batch[0]->ke->spec.zouts.empty()) {
+    // records that are too large for one launch: the batch in two parts
+    const size_t PB = batch[0]->ke->spec.part_bytes;
+    size_t bytes = 0;
+    for (Task* t : batch) {
+      t->chunking(0);
+      bytes += (size_t)t->nchunks * PB;
+    }
+    void* parts = nullptr;
+    if (bytes <= kZonalRecordBytes) {
+      try { parts = store.alloc(bytes); } catch (const std::exception&) {}
+    }
+    if (!parts) {
+      const auto mid = batch.begin() + batch.size() / 2;
+      run_batch({batch.begin(), mid}, async);
+      run_batch({mid, batch.end()}, async);
+      return;
+    }
+    try {
+      launch_batch(batch, parts, async);
+    } catch (...) {
+      store.release(parts);
+      throw;
+    }
+    return;
+  }
+  launch_batch(batch, nullptr, async);
+}
+
+// `parts`: the records of a batch of several tasks, null otherwise.
+void Runtime::launch_batch(const std::vector<Task*>& batch, void* parts, std::vector<Readback>* async) {
   HostTimer ht_launch(cnt.ms_launch);
   const KernelEntry& ke = *batch[0]->ke;
   const KernelSpec& ks = ke.spec;
@@ -1422,7 +1478,7 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
   if (opt.form == FORM_PLAIN) {
     for (Task* t : batch) {
       t->chunking(opt.chunk_tiles > 0 ? opt.chunk_tiles : 1);  // one block per launch: every tile its own chunk
-      void* parts = zonal ? store.alloc((size_t)t->nchunks * ks.part_bytes) : nullptr;
+      parts = zonal ? zonal_records(*t) : nullptr;
       std::vector<std::pair<uint32_t, int>> order;
       for (int b = 0; b < t->L.NB0 * t->L.NB1; b++) order.push_back({morton2(b % t->L.NB0, b / t->L.NB0), b});
       std::sort(order.begin(), order.end());
@@ -1445,7 +1501,7 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
     const bool q = opt.queue == 1;
     if (opt.chunk_tiles > 0 || zonal) t->chunking(opt.chunk_tiles);
     else t->chunking_static(gmax);
-    void* parts = zonal ? store.alloc((size_t)t->nchunks * ks.part_bytes) : nullptr;
+    parts = zonal ? zonal_records(*t) : nullptr;
     launch(t->args, t->L, nul, nul, 1, t->nchunks, q ? queue() : nul, parts, grid_for(t->nchunks));
     if (zonal) {
       fold_results(batch, parts, nullptr, nullptr, t->nchunks, async);
@@ -1479,7 +1535,6 @@ void Runtime::run_batch(const std::vector<Task*>& batch, std::vector<Readback>* 
   char* dtab = (char*)device_table(tab);
   void* tasks_dev = dtab;
   void* starts_dev = dtab + (size_t)T * ks.task_size;
-  void* parts = zonal ? store.alloc((size_t)total * ks.part_bytes) : nullptr;
   HostLaunch L0{};
   std::vector<char> a0(ks.args_size, 0);
   launch(a0, L0, tasks_dev, starts_dev, T, total, q ? queue() : nul, parts, grid_for(total));

@@ -197,6 +197,8 @@ class Runtime {
   int predict(const std::vector<Node*>& targets);
   Variant access_value(Node* n);
   void run_batch(const std::vector<Task*>& batch, std::vector<Readback>* async);
+  void launch_batch(const std::vector<Task*>& batch, void* parts, std::vector<Readback>* async);
+  void* zonal_records(Task& t);
   void fold_results(const std::vector<Task*>& batch, void* parts, void* tasks_dev, void* starts_dev, int maxn,
                     std::vector<Readback>* async);
   void distribute(Readback& rb);

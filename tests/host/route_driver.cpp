@@ -1,6 +1,7 @@
 // Which kernels the runtime compiles and launches, and what memory it takes for them, on the
 // device double (dev_double.cpp, compiled into this file behind hooks on its compilation, launch
 // and allocation entries) through the C ABI. One scenario per run: route_driver NAME.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -16,9 +17,11 @@
 
 #define function function_double
 #define launch launch_double
+#define malloc_device malloc_device_double
 #define spread spread_double
 #include "dev_double.cpp"
 #undef spread
+#undef malloc_device
 #undef function
 #undef launch
 
@@ -32,11 +35,16 @@ struct Launched {
 std::vector<std::string> compiled;  // kernels asked for, in order
 std::map<std::string, std::string> sources;
 std::vector<Launched> launched;
+size_t largest = 0;  // device allocation
 std::function<void(const Launched&, void**, const size_t*, int)> on_launch;
 }  // namespace
 
 namespace mapx {
 namespace dev {
+void* malloc_device(size_t bytes) {
+  largest = std::max(largest, bytes);
+  return malloc_device_double(bytes);
+}
 Function function(const std::string& source, const std::string& name) {
   compiled.push_back(name);
   sources[name] = source;
@@ -186,6 +194,48 @@ void scenario_served_plan() {
   expect(launches("_pack") == 1 && launches("_step") == 5, "the plan of a served request has no chain");
 }
 
+// Per-zone statistics: the partial records of chunks (24 bytes a zone) stay below what the cells take.
+R statistics(int w, int h, int nz, bool windows) {
+  R a = input(w, h, 256, F32, 4), z = input(w, h, 256, S32, 4);
+  eval({a, z});
+  return R(ma_zonalStats(windows ? conv(a, {1, 2, 1, 2, 4, 2, 1, 2, 1}).n : a.n, z.n, nz));
+}
+void scenario_zone_records() {
+  ma_setOption("focal_zonal", 1);
+  int chunks = 0;
+  on_launch = [&](const Launched& l, void** params, const size_t*, int n) {
+    if (n == 8 && has(l.name, "krn_") && !ends(l.name, "_fin")) chunks = *(int*)params[5];
+  };
+  struct { int w, h, nz, windows, least, most; } one[] = {
+      {4096, 4096, 16, 1, 2048, 2048}, {4096, 4096, 3000, 1, 256, 256}, {2048, 2048, 3000, 1, 256, 256},
+      {2048, 2048, 256, 1, 1024, 1024}, {4096, 4096, 256, 0, 512, 512}, {512, 512, 3000, 0, 64, 64}, {100, 60, 3000, 1, 1, 15}};
+  for (auto& c : one) {
+    eval({statistics(c.w, c.h, c.nz, c.windows != 0)});
+    expect(chunks >= c.least && chunks <= c.most, std::to_string(chunks) + " chunks of " + std::to_string(c.w) + " x " +
+           std::to_string(c.h) + " cells, " + std::to_string(c.nz) + " zones");
+  }
+  // a batch whose records are more than 512 MB goes in several launches
+  largest = 0;
+  launched.clear();
+  std::vector<R> v;
+  for (int i = 0; i < 160; i++) v.push_back(statistics(512 - i % 16, 512 - i / 16, 3000, false));
+  eval(v);
+  expect(largest <= (size_t)512 << 20, "one allocation of " + std::to_string(largest >> 20) + " MB");
+  expect((int)launched.size() <= 2 * 2 * 3, "the batch in too many launches");
+  on_launch = nullptr;
+}
+// Where the device is too small for these records, coarser chunks are taken.
+void scenario_zone_records_small_device() {
+  ma_setOption("focal_zonal", 1);
+  setenv("MAPX_DOUBLE_HBM", std::to_string(20 << 20).c_str(), 1);
+  eval({statistics(1024, 1024, 3000, true)});
+  std::vector<R> v;
+  for (int i = 0; i < 6; i++) v.push_back(statistics(256 - i, 256, 3000, false));
+  setenv("MAPX_DOUBLE_HBM", std::to_string(16 << 20).c_str(), 1);
+  eval(v);
+  unsetenv("MAPX_DOUBLE_HBM");
+}
+
 // A served flow accumulation is admitted with the memory it takes: its raster and the scan's scratch.
 void scenario_served_flow() {
   for (auto& c : std::vector<std::pair<int, int>>{{40, 30}, {700, 500}}) {
@@ -239,7 +289,9 @@ void scenario_no_bits() {
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> all = {{"compile", scenario_compile}, {"served plan", scenario_served_plan}, {"no bits", scenario_no_bits},
-                                                      {"served flow", scenario_served_flow}};
+                                                      {"served flow", scenario_served_flow},
+                                                      {"zone records", scenario_zone_records},
+                                                      {"zone records, small device", scenario_zone_records_small_device}};
   if (argc != 2 || !all.count(argv[1])) return 3;
   ma_setupDevices("", DEV_GPU, "");
   all.at(argv[1])();

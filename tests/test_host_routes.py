@@ -21,7 +21,7 @@ def driver():
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["compile", "served plan", "no bits", "served flow"])
+@pytest.mark.parametrize("scenario", ["compile", "served plan", "no bits", "served flow", "zone records", "zone records, small device"])
 def test_routes(driver, scenario):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0", UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
     r = subprocess.run([driver, scenario], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300, env=env, cwd="/tmp")
