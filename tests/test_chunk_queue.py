@@ -1,9 +1,12 @@
 """The chunk queue of the generated kernels (device/mapx_dev.hiph, work distribution): its device text compiled for
 the host, a work-group a thread-0 at a time in random order. A take takes effect when its result is used, the last
 one of a work-group, whose result nobody uses, as late as it can: launch after launch every chunk has to be dealt
-out once and the queue to be left at zero."""
+out once and the queue to be left at zero. On the GPU, statistics of a batch against its rasters alone."""
 import os
 import subprocess
+
+import numpy as np
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "map_amd", "csrc", "device", "mapx_dev.hiph")
@@ -37,7 +40,7 @@ static void atomicExch(u32* p, u32 v) { *p = v; }
 static void __syncthreads() {}
 static int readfirstlane(int v) { return v; }
 #define __builtin_amdgcn_readfirstlane readfirstlane
-static void landed(u32) { land(); }
+static void landed() { land(); }
 @SECTION@
 int main(int argc, char** argv) {
   const int grid = atoi(argv[1]), n = atoi(argv[2]);
@@ -84,3 +87,28 @@ def test_queue_deals_every_chunk_once_launch_after_launch(tmp_path):
     for grid in (8, 16, 256):
         for n in (1, 7, 8, 9, 100, 4095, 4096, 4099, 20000):
             assert subprocess.run([str(exe), str(grid), str(n)], timeout=60).returncode == 0, (grid, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,side", [(6, 2000), (9, 300)])  # more than 4096 chunks (dealt out in runs of eight), and fewer
+def test_batches_match_single_rasters(G, n, side):
+    """Statistics of whole numbers (every sum exact) of rasters that go in one launch with the queue, evaluated twice."""
+    rng = np.random.Generator(np.random.PCG64(n))
+    outs, want = [], []
+    for i in range(n):
+        print("case batch", n, side, i, flush=True)
+        h, w = side - 3 * i, side + 5 * i
+        v = rng.integers(-100, 101, (h, w)).astype(np.float32)
+        z = ((np.arange(w)[None] // 31 + np.arange(h)[:, None] // 17) % 16).astype(np.int32)
+        R, Z = G.from_array(v, (512, 512)), G.from_array(z, (512, 512))
+        alone = G.zstats(R + 0.0, Z, 16)
+        G.eval(alone)
+        want.append((alone.table(), np.bincount(z.ravel()), np.bincount(z.ravel(), v.ravel())))
+        outs.append(G.zstats(R, Z, 16))
+    for again in range(2):
+        G.eval(*outs)
+        for s, (t, count, total) in zip(outs, want):
+            got = s.table()
+            assert np.array_equal(got["count"], count) and np.array_equal(got["sum"], total)
+            for k in ("sum", "min", "max", "count"):
+                assert np.array_equal(got[k], t[k])
