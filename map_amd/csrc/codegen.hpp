@@ -73,9 +73,9 @@ struct KernelSpec {
 // write to HBM (group outputs consumed later, written to files or requested).
 // `libm`: FP32 sqrt, atan2 and sin/cos pairs call the device library instead of
 // the fast paths of mapx_dev.hiph (mx::sqrt_f32, mx::atan2_f32, mx::sincos_f32).
+KernelSpec generate_kernel(const Group& g, const std::vector<Node*>& d2_outs, TileShape tile, bool libm = false);
 // Work-groups a slice of partial records is folded by: one per 16 zones.
 int fold_groups(const KernelSpec& ks);
-KernelSpec generate_kernel(const Group& g, const std::vector<Node*>& d2_outs, TileShape tile, bool libm = false);
 
 // The group's nodes in the kernel's local numbering: inputs (D2, then D0,
 // each by id), then the group's nodes by id.

@@ -19,11 +19,13 @@
 // before the columns, its results stored after them to `out` (block-tiled, like
 // every raster), from which the next band reads its starting column.
 //
-// What bounds it: the chain of columns. A column is 2 rows x 20 instructions in
-// a wavefront, about 260 cycles of dependent ones, and a launch of a large raster
-// has about one wavefront per SIMD. (One launch for all bands, with wavefronts
-// that wait for the row before theirs, took as long: each hand-over costs what
-// 16 columns do.)
+// What bounds it: the latencies of a launch, which with about one wavefront per
+// SIMD nothing overlaps. Of a band's 18.5 us (16384^2 cells) the chain of columns
+// is 5.7: 2 rows x 20 instructions a column, some 210 cycles of dependent ones. The
+// other 12.9 are the launch itself, the loads before the first column and the stores
+// after the last (measured with the columns left out). (One launch for all bands, with
+// wavefronts that wait for the row before theirs, took as long: each hand-over costs
+// what 16 columns do.)
 // The division of the interpolation weight, d1/d0, is by a number that all rows
 // of a column share: q = d1 * (1/d0), then q + (d1 - q d0) * (1/d0) with fused
 // multiply-adds is the correctly rounded quotient (Markstein, IBM Journal of
