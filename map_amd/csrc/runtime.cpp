@@ -1514,11 +1514,13 @@ void Runtime::launch_batch(const std::vector<Task*>& batch, void* parts, std::ve
   const int T = (int)batch.size();
   std::vector<int> starts(T + 1, 0);
   int maxn = 0;
-  long tiles_total = 0;
-  for (Task* t : batch) tiles_total += t->tiles();
-  const int ch = opt.chunk_tiles > 0 ? opt.chunk_tiles : adaptive_chunk(tiles_total, gmax);
+  if (!zonal) {  // (zonal tasks keep their chunks: run_batch has counted them)
+    long tiles_total = 0;
+    for (Task* t : batch) tiles_total += t->tiles();
+    const int ch = opt.chunk_tiles > 0 ? opt.chunk_tiles : adaptive_chunk(tiles_total, gmax);
+    for (Task* t : batch) t->chunking(ch);
+  }
   for (int i = 0; i < T; i++) {
-    batch[i]->chunking(ch);
     starts[i + 1] = starts[i] + batch[i]->nchunks;
     maxn = std::max(maxn, batch[i]->nchunks);
   }
